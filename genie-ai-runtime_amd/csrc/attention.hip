@@ -11,15 +11,9 @@
 // sliding window, positions < seq - window are excluded (they contribute
 // exactly zero in the reference).
 //
-// Prefill (flash_attention_prefill_batched_kernel, attention.cu:382-514)
-// is the same computation per query token t with the causal bound
-// seq = start_pos + t + 1: grid z runs over blocks of tq tokens, one split
-// each; a wave's MFMA columns are its tq tokens x G heads (each column with
-// its own causal bound, so a K/V tile read once serves all of them) and the
-// wave writes the normalised outputs directly (no partials, no reduce); a
-// decode call with a single split does the same for its one token.
+// The prefill (several query tokens) is attention_prefill.hip.
 //
-// MI355X mapping: one wave64 per (KV head, split[, token]) computes ALL
+// MI355X mapping: one wave64 per (KV head, split) computes ALL
 // query heads of its GQA group, so each KV byte is read from HBM once.
 // Keys go in 32-key tiles held in registers (the next tile's rows load
 // while the current one is computed).  Q.K^T runs on the matrix cores
@@ -27,16 +21,14 @@
 // needs one cross-lane step); the V tile is transposed by an identity MFMA
 // (int8: v_mfma_i32_32x32x32_i8 against I, exact) and P.V runs as
 // v_mfma_f32_32x32x16_f16 with the fp32 probabilities (times vs) split into
-// a high and a low fp16 part, so the P.V products keep ~22 bits: in decode
-// the two parts are extra rows of the A operand (2 x G rows), in prefill two
-// A operands accumulating into the same rows, so a prefill wave serves 32
-// columns (8 tokens x 4 heads).
+// a high and a low fp16 part, as extra rows of the A operand (2 x G rows), so
+// the P.V products keep ~22 bits.
 #include <float.h>
 #include <stdlib.h>
 #include <string.h>
 #include "kq_common.h"
 #include "attention.h"
-#include "quant_chunk.h"
+#include "attn_common.h"
 
 #ifndef ATTN_RED_XCD
 #define ATTN_RED_XCD 1
@@ -44,15 +36,6 @@
 
 namespace jllm_hip {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4a __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2a __attribute__((ext_vector_type(2)));
-typedef float f32x4a __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int AT_KEYS = 32;          // keys per tile (one MFMA column block)
 // LDS row stride of the P' tile (halves): 18 dwords, so the 8-byte writes
 // and reads of lanes (row li, key group lg) spread evenly over the 32 banks
 // (a 16-dword stride put every row on the same 4 banks)
@@ -60,28 +43,6 @@ constexpr int AT_PLD = AT_KEYS + 4;
 constexpr int AT_MAXHD = 128;
 constexpr int AT_MAXG = 16;          // max query heads per KV head
 constexpr int AT_MAXS = ATTN_MAX_SPLITS;   // max splits
-
-// 4 signed int8 (one word) -> 4 exact fp16 values (two words): with u = b ^ 0x80
-// in [1, 255], the half with bits 0x64 : u is 1024 + u (byte permutes against
-// a word of 0x64 bytes), minus 1152 gives b.
-__device__ __forceinline__ u32x2a i8x4_to_h4(uint32_t w) {
-    const half2_t bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const uint32_t u = w ^ 0x80808080u;
-    const uint32_t a = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
-    const uint32_t b = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
-    return u32x2a{h2_bits(as_h2(a) + bias), h2_bits(as_h2(b) + bias)};
-}
-
-template <bool INT8>
-__device__ __forceinline__ h8 kv8_to_h8(const uint8_t* p) {
-    if (INT8) {
-        const u32x2a w = *(const u32x2a*)p;
-        const u32x2a lo = i8x4_to_h4(w.x), hi = i8x4_to_h4(w.y);
-        return __builtin_bit_cast(h8, u32x4a{lo.x, lo.y, hi.x, hi.y});
-    } else {
-        return __builtin_bit_cast(h8, *(const u32x4a*)p);
-    }
-}
 
 #ifdef JLLM_ATTN_TRACE
 // probe builds only: per-wave timestamps (s_memrealtime, 100 MHz) of the last
@@ -133,43 +94,33 @@ size_t attn_scratch_bytes(int n_heads, int n_splits, int head_dim) {
 }
 
 // LDS of one wave (P' tile, per-key scales, then its final hi/lo rows)
-__host__ __device__ size_t attn_wave_lds_bytes(int n_heads, int n_kv, int head_dim, int tq) {
-    const int G = n_heads / n_kv * tq;                                // columns of a wave
-    const bool ps = tq > 1;                                          // prefill: one row per column
-    const size_t loop = (size_t)(ps ? 64 : 32) * AT_PLD * 2 + 96 * 4; // P' rows (fp16) + corr/ks/vs
-    // final rows (fp32, >= 8); prefill: all 32 rows of the accumulator layout,
-    // so the epilogue stores them without a per-row predicate
-    const size_t outb = (size_t)(ps ? 32 : ((2 * G + 7) & ~7)) * head_dim * 4;
+__host__ __device__ size_t attn_wave_lds_bytes(int n_heads, int n_kv, int head_dim) {
+    const int G = n_heads / n_kv;
+    const size_t loop = (size_t)32 * AT_PLD * 2 + 96 * 4;            // P' rows (fp16) + corr/ks/vs
+    const size_t outb = (size_t)((2 * G + 7) & ~7) * head_dim * 4;    // final rows (fp32, >= 8)
     return ((loop > outb ? loop : outb) + 15) & ~(size_t)15;
 }
-// a workgroup of W waves: W wave regions, then (m, l) of each wave's columns
-__host__ __device__ size_t attn_lds_bytes(int n_heads, int n_kv, int head_dim, int tq, int W) {
-    return (size_t)W * attn_wave_lds_bytes(n_heads, n_kv, head_dim, tq) +
+// a workgroup of W waves: W wave regions, then (m, l) of each wave's heads
+__host__ __device__ size_t attn_lds_bytes(int n_heads, int n_kv, int head_dim, int W) {
+    return (size_t)W * attn_wave_lds_bytes(n_heads, n_kv, head_dim) +
            (W > 1 ? (size_t)W * 2 * 32 * 4 + (size_t)(ATTN_MAX_WAVES + 1) * 32 * 4 + (size_t)W * 32 * 4 : 0);
 }
 
-// One wave per (KV head, split[, block of tq query tokens]).  The wave's
-// "columns" are its (token, head) pairs: column c = token tok0 + c / G, head
-// kvh * G + c % G, GC = tq * G <= 32 of them; each has its own causal bound
-// (and window), so one key tile serves tq tokens.  Lane (li = lane & 31,
-// lg = lane >> 5); below, "head li" means column li.
+// One wave per (KV head, split), all G query heads of the KV head.  Lane (li =
+// lane & 31, lg = lane >> 5); below, "head li" means head kvh * G + li.
 //   Q.K^T : C = K.q^T (rows = the tile's 32 keys, cols = query heads, K = d);
 //           lane group lg covers d in [lg*hd/2, (lg+1)*hd/2), 8 at a time
 //   V^T   : the V rows are turned into columns on the matrix cores: with A =
 //           V rows (K = d) and B = the identity, C = V lands in the MFMA
 //           output layout, i.e. lane (d = li, lg) holds 16 keys of column d
 //           (int8: one v_mfma_i32_32x32x32_i8 per 32 d, exact)
-//   P.V   : A = P'  (decode: rows = heads, high parts then low parts;
-//           prefill: rows = columns, the high and the low parts as two A
-//           operands into the same accumulator; K = keys in the order the
-//           transpose delivers them), B = those V columns
+//   P.V   : A = P'  (rows = heads, high parts then low parts; K = keys in the
+//           order the transpose delivers them), B = those V columns
 // The K and V rows of the next tile are loaded into registers while the
 // current tile is computed.
-// MT: several query tokens per wave (per-column causal bounds); the
-// single-token form (decode, or tq == 1) compiles without the column masks.
-// G4: at most 4 columns (decode with <= 4 q heads per KV head): the P.V rows
+// G4: at most 4 q heads per KV head: the P.V rows
 // 8 and up hold nothing, so their accumulators are never rescaled.
-template <bool INT8, int HD, bool MT, bool G4>
+template <bool INT8, int HD, bool G4>
 __global__ __launch_bounds__(64 * ATTN_MAX_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_partial_kernel(AttnArgs a) {
     constexpr int EB = INT8 ? 1 : 2;
@@ -178,34 +129,19 @@ void attn_partial_kernel(AttnArgs a) {
     constexpr int NDT = HD / 32;                        // 32-wide d chunks
     constexpr int VW = NDT * EB;                        // V: 16-byte chunks per lane
     constexpr int NST = half / 8;                       // Q.K^T MFMA steps
-    // prefill (MT): the high and low fp16 parts of P' are two A operands
-    // accumulating into the same accumulator row, one row per column, so a
-    // wave serves 32 columns; decode keeps a row for each (2 x G rows)
-    constexpr bool PS = MT;
-    constexpr int PROWS = PS ? 64 : 32;                 // P' tile rows in LDS
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_wg[];
     const int W = a.wsplit;
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const size_t wave_lds = attn_wave_lds_bytes(a.n_heads, a.n_kv, a.head_dim, a.tq);
+    const size_t wave_lds = attn_wave_lds_bytes(a.n_heads, a.n_kv, a.head_dim);
     uint8_t* smem = smem_wg + (size_t)wv * wave_lds;
     uint64_t tr[4] = {0, 0, 0, 0};
     AT_MARK(0);
-    // prefill: the last token blocks (the most key tiles) are dispatched first
     const int kvh = blockIdx.x, split = blockIdx.y;
-    const int tok0 = MT ? ((int)gridDim.z - 1 - (int)blockIdx.z) * a.tq : blockIdx.z;
-    const int aseq = (!MT && a.pos_dev) ? __builtin_amdgcn_readfirstlane(*a.pos_dev) + 1 : a.seq;
+    const int seq = a.pos_dev ? __builtin_amdgcn_readfirstlane(*a.pos_dev) + 1 : a.seq;
     const int G = a.n_heads / a.n_kv;
-    const int ntok = MT ? min(a.tq, a.tokens - tok0) : 1;       // tokens of this wave
-    const int GC = ntok * G;                                    // live columns
     const int l = (int)threadIdx.x & 63, li = l & 31, lg = l >> 5;
-    // column li: its token, causal bound and window start
-    const int ctok = MT ? tok0 + (li < GC ? li / G : 0) : tok0;
-    const int seq_c = aseq + ctok;
-    const int lo_c = a.window > 0 ? max(0, seq_c - a.window) : 0;
-    // the wave's key range covers every column's
-    const int seq = aseq + tok0 + ntok - 1;
     const int kv_dim = a.n_kv * a.cache_head_dim, hoff = kvh * a.cache_head_dim;
-    const int lo_pos = a.window > 0 ? max(0, aseq + tok0 - a.window) : 0;
+    const int lo_pos = a.window > 0 ? max(0, seq - a.window) : 0;
     const int span = seq - lo_pos;
     const int S = a.n_splits;
     const int per = (span + S - 1) / S;
@@ -243,37 +179,25 @@ void attn_partial_kernel(AttnArgs a) {
     __builtin_amdgcn_sched_barrier(0);
 
     _Float16* sP = (_Float16*)smem;                              // [32 rows][AT_PLD: 32 keys + pad]
-    float* sMisc = (float*)(smem + PROWS * AT_PLD * 2);         // corr[32] | ks[32] | vs[32]
+    float* sMisc = (float*)(smem + 32 * AT_PLD * 2);         // corr[32] | ks[32] | vs[32]
 
     // q operand: lane (head li, lg), step st -> d = lg*half + 8*st + [0, 8)
-    // (every lane loads a valid row -- its column's head modulo G -- so the
-    // loads issue unpredicated; lanes without a column then zero theirs)
+    // (every lane loads a valid row -- its head modulo G -- so the loads issue
+    // unpredicated; lanes without a head then zero theirs)
     h8 qa[NST];
 #pragma unroll
     for (int st = 0; st < NST; st++) {
-        const u32x4a qv = *(const u32x4a*)(a.q + (int64_t)ctok * a.n_heads * hd + (int64_t)(kvh * G + li % G) * hd +
+        const u32x4a qv = *(const u32x4a*)(a.q + (int64_t)(kvh * G + li % G) * hd +
                                            lg * half + 8 * st);
-        qa[st] = __builtin_bit_cast(h8, li < GC ? qv : u32x4a{0u, 0u, 0u, 0u});
+        qa[st] = __builtin_bit_cast(h8, li < G ? qv : u32x4a{0u, 0u, 0u, 0u});
     }
-    for (int i = l; i < PROWS * AT_PLD; i += 64) sP[i] = (_Float16)0.0f;
+    for (int i = l; i < 32 * AT_PLD; i += 64) sP[i] = (_Float16)0.0f;
 
-    // identity operands of the V transpose.  int8: lane (col li, lg) holds
-    // B[16lg + i][li] = (16lg + i == li).  fp16: two K = 16 halves, lane
-    // (col li, lg) holds B_hh[8lg + e][li] = (16hh + 8lg + e == li).
     i32x4 eye8;
     h8 eyeh[2];
-    {
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        const int pos = li - 16 * lg;
-        if (pos >= 0 && pos < 16) w[pos >> 2] = 1u << (8 * (pos & 3));
-        eye8 = i32x4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) eyeh[hh][e] = (_Float16)((16 * hh + 8 * lg + e == li) ? 1.0f : 0.0f);
-    }
+    eye_operands(li, lg, eye8, eyeh);
 
-    // running softmax state of column li (meaningful in lanes li < GC; both
+    // running softmax state of head li (meaningful in lanes li < G; both
     // lane halves keep identical copies)
     float run_m = -FLT_MAX, run_l = 0.0f;
     f32x16 acc[NDT];
@@ -306,24 +230,17 @@ void attn_partial_kernel(AttnArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; r++) { kscl[4 * m4 + r] = k4[r]; vscl[4 * m4 + r] = v4[r]; }
         }
-        // 2. online softmax for column li (lanes li < GC do the useful work)
+        // 2. online softmax for head li (lanes li < G do the useful work)
         float mx = -FLT_MAX;
 #pragma unroll
         for (int vv = 0; vv < 16; vv++) sc[vv] *= kscl[vv];
-        // key masks only where a tile can hold dead keys (uniform branch): a
-        // prefill tile that reaches past the first column's causal bound or
-        // below the last column's window start, or a tile of fewer than
-        // AT_KEYS keys (a live key keeps its score either way, so skipping
-        // the masks of a full tile changes no bit)
-        const bool full = n == AT_KEYS && (!MT || (p0 + AT_KEYS <= aseq + tok0 &&
-                                                   (a.window <= 0 || p0 >= aseq + tok0 + ntok - 1 - a.window)));
-        if (!full) {
+        // key masks only on a tile of fewer than AT_KEYS keys (uniform branch; a
+        // live key keeps its score either way)
+        if (n < AT_KEYS) {
 #pragma unroll
             for (int vv = 0; vv < 16; vv++) {
                 const int key = 8 * (vv >> 2) + 4 * lg + (vv & 3);
-                const int pos = p0 + key;
-                const bool live = MT ? (key < n && pos < seq_c && pos >= lo_c) : key < n;
-                sc[vv] = live ? sc[vv] : -INFINITY;
+                sc[vv] = key < n ? sc[vv] : -INFINITY;
             }
         }
 #pragma unroll
@@ -354,16 +271,16 @@ void attn_partial_kernel(AttnArgs a) {
         }
         run_l = run_l * corr + ps;
         run_m = m_new;
-        // no live column's maximum moved: every rescale factor is exactly 1
+        // no head's maximum moved: every rescale factor is exactly 1
         // (e^0), so the accumulators keep their values without the multiply
-        const bool rescale = __builtin_amdgcn_ballot_w64(li < GC && corr != 1.0f) != 0;
-        if (li < GC) {
+        const bool rescale = __builtin_amdgcn_ballot_w64(li < G && corr != 1.0f) != 0;
+        if (li < G) {
             // keys 8m + 4lg + [0,4) for m = 0..3: four consecutive keys per 8-byte store
 #pragma unroll
             for (int m4 = 0; m4 < 4; m4++) {
                 const int key0 = 8 * m4 + 4 * lg;
                 *(u32x2a*)&sP[li * AT_PLD + key0] = u32x2a{hi2[2 * m4], hi2[2 * m4 + 1]};
-                *(u32x2a*)&sP[((PS ? 32 : GC) + li) * AT_PLD + key0] = u32x2a{lo2[2 * m4], lo2[2 * m4 + 1]};
+                *(u32x2a*)&sP[(G + li) * AT_PLD + key0] = u32x2a{lo2[2 * m4], lo2[2 * m4 + 1]};
             }
             if (lg == 0) sMisc[li] = corr;
         }
@@ -377,7 +294,7 @@ void attn_partial_kernel(AttnArgs a) {
 #pragma unroll
         for (int vv = 0; vv < NLIVE; vv++) {
             const int r = 8 * (vv >> 2) + 4 * lg + (vv & 3);
-            cr[vv] = PS ? (r < GC ? sMisc[r] : 1.0f) : (r < 2 * GC ? sMisc[r < GC ? r : r - GC] : 1.0f);
+            cr[vv] = r < 2 * G ? sMisc[r < G ? r : r - G] : 1.0f;
         }
         if (rescale) {
 #pragma unroll
@@ -385,17 +302,12 @@ void attn_partial_kernel(AttnArgs a) {
 #pragma unroll
                 for (int vv = 0; vv < NLIVE; vv++) acc[dt][vv] *= cr[vv];
         }
-        h8 pa[2], pl[2];
+        h8 pa[2];
 #pragma unroll
         for (int st = 0; st < 2; st++) {
             const u32x2a lo4 = *(const u32x2a*)&sP[li * AT_PLD + 16 * st + 4 * lg];
             const u32x2a hi4 = *(const u32x2a*)&sP[li * AT_PLD + 16 * st + 8 + 4 * lg];
             pa[st] = __builtin_bit_cast(h8, u32x4a{lo4.x, lo4.y, hi4.x, hi4.y});
-            if (PS) {
-                const u32x2a a4 = *(const u32x2a*)&sP[(32 + li) * AT_PLD + 16 * st + 4 * lg];
-                const u32x2a b4 = *(const u32x2a*)&sP[(32 + li) * AT_PLD + 16 * st + 8 + 4 * lg];
-                pl[st] = __builtin_bit_cast(h8, u32x4a{a4.x, a4.y, b4.x, b4.y});
-            }
         }
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
@@ -424,7 +336,6 @@ void attn_partial_kernel(AttnArgs a) {
                         vb[e + 1] = h2[1];
                     }
                     acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pa[st], vb, acc[dt], 0, 0, 0);
-                    if (PS) acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pl[st], vb, acc[dt], 0, 0, 0);
                 }
             }
         }
@@ -456,229 +367,123 @@ void attn_partial_kernel(AttnArgs a) {
     // 4. S == 1: the normalised output straight from this wave; else the
     //    unnormalised partials m, l per head (acc = high rows + low rows)
     const int pbase = kvh * G;
-    float* sO = (float*)smem;                                  // [2G][hd]
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
-    if constexpr (!MT) {
-        // decode: the rows go to LDS transposed, sOT[d][R] (R = 2G rounded up
-        // to 8), four consecutive rows of a column per 16-byte store, only the
-        // row groups that hold a head; then lane l forms the outputs of
-        // d = l, l + 64, ... for every head (high + low row) and stores them
-        // coalesced along d
-        const int R = (2 * G + 7) & ~7;
-        float* sOT = (float*)smem;
-#pragma unroll
-        for (int dt = 0; dt < NDT; dt++) {
-#pragma unroll
-            for (int m4 = 0; m4 < 4; m4++) {
-                if (8 * m4 >= 2 * G) break;
-                *(f32x4a*)&sOT[(32 * dt + li) * R + 8 * m4 + 4 * lg] =
-                    f32x4a{acc[dt][4 * m4], acc[dt][4 * m4 + 1], acc[dt][4 * m4 + 2], acc[dt][4 * m4 + 3]};
-            }
-        }
-        __builtin_amdgcn_s_waitcnt(0xc07f);
-        __builtin_amdgcn_wave_barrier();
-        if (W > 1) {
-            // combine the W waves' states per head, waves in order:
-            // M = max_w m_w, num = sum_w acc_w e^(m_w - M), den = sum_w l_w e^(m_w - M);
-            // the workgroup's output (S == 1) or its partial (M, den, num).
-            // Wave weights e^(m_w - M) are formed once per (wave, head), then
-            // every thread issues all its LDS reads before it adds.
-            float* sML = (float*)(smem_wg + (size_t)W * wave_lds);     // [W][m[32] | l[32]], then f [W][32]
-            float* sF = sML + W * 64;
-            if (lg == 0) { sML[wv * 64 + li] = run_m; sML[wv * 64 + 32 + li] = run_l; }
-            __syncthreads();
-            const int t = (int)threadIdx.x;
-            if (t < W * G) {
-                const int u = t / G, h = t % G;
-                float M = -FLT_MAX;
-                for (int w = 0; w < W; w++) M = fmaxf(M, sML[w * 64 + h]);
-                sF[u * 32 + h] = expf(sML[u * 64 + h] - M);
-                if (u == 0) sF[ATTN_MAX_WAVES * 32 + h] = M;
-            }
-            __syncthreads();
-            float* pm = a.part;
-            float* pl = a.part + (int64_t)a.n_heads * S;
-            float* pacc = a.part + (int64_t)a.n_heads * S * 2;
-            for (int e = t; e < G * hd; e += 64 * W) {
-                const int d = e / G, h = e % G;     // lanes: consecutive heads of one d, then d
-                float hi[ATTN_MAX_WAVES], lo[ATTN_MAX_WAVES], f[ATTN_MAX_WAVES], lv[ATTN_MAX_WAVES];
-#pragma unroll
-                for (int u = 0; u < ATTN_MAX_WAVES; u++) {
-                    if (u < W) {
-                        const float* so = (const float*)(smem_wg + (size_t)u * wave_lds);
-                        hi[u] = so[d * R + h];
-                        lo[u] = so[d * R + G + h];
-                        f[u] = sF[u * 32 + h];
-                        lv[u] = sML[u * 64 + 32 + h];
-                    }
-                }
-                float num = 0.0f, den = 0.0f;
-#pragma unroll
-                for (int u = 0; u < ATTN_MAX_WAVES; u++) {
-                    if (u < W) {
-                        num += (hi[u] + lo[u]) * f[u];
-                        den += lv[u] * f[u];
-                    }
-                }
-                if (S == 1) {
-                    a.out[(int64_t)(pbase + h) * hd + d] = f32_to_f16_bits(den > 0.0f ? num / den : 0.0f);
-                } else {
-                    pacc[((int64_t)(pbase + h) * S + split) * hd + d] = num;
-                    if (d == 0) {
-                        pm[(int64_t)(pbase + h) * S + split] = sF[ATTN_MAX_WAVES * 32 + h];
-                        pl[(int64_t)(pbase + h) * S + split] = den;
-                    }
-                }
-            }
-#ifdef JLLM_ATTN_TRACE
-            AT_MARK(3);
-            {
-                const int gw = ((int)blockIdx.y * (int)gridDim.x + (int)blockIdx.x) * W + wv;
-                if (l < 4 && gw < 8192) {
-                    uint64_t tv = 0;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) if (l == i) tv = tr[i];
-                    g_attn_trace[gw * 4 + l] = tv;
-                }
-            }
-#endif
-            return;
-        }
-        if (S == 1) {
-            const float inv_l = run_l > 0.0f ? 1.0f / run_l : 0.0f;
-            for (int h = 0; h < G; h++) {
-                const float il = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv_l), h));
-                uint16_t* ot = a.out + (int64_t)(pbase + h) * hd;
-                for (int d = l; d < hd; d += 64)
-                    ot[d] = f32_to_f16_bits((sOT[d * R + h] + sOT[d * R + G + h]) * il);
-            }
-            return;
-        }
-        float* pm = a.part;
-        float* pl = a.part + (int64_t)a.n_heads * S;
-        if (li < G && lg == 0) {
-            pm[(int64_t)(pbase + li) * S + split] = run_m;
-            pl[(int64_t)(pbase + li) * S + split] = run_l;
-        }
-        float* pacc = a.part + (int64_t)a.n_heads * S * 2 + ((int64_t)pbase * S + split) * hd;
-        for (int h = 0; h < G; h++) {
-            for (int d = l; d < hd; d += 64) pacc[(int64_t)h * S * hd + d] = sOT[d * R + h] + sOT[d * R + G + h];
-        }
-#ifdef JLLM_ATTN_TRACE
-        AT_MARK(3);
-        const int gw = blockIdx.y * gridDim.x + blockIdx.x;
-        if (l < 4 && gw < 8192) {
-            uint64_t tv = 0;
-#pragma unroll
-            for (int i = 0; i < 4; i++) if (l == i) tv = tr[i];
-            g_attn_trace[gw * 4 + l] = tv;
-        }
-#endif
-        return;
-    }
+    // decode: the rows go to LDS transposed, sOT[d][R] (R = 2G rounded up
+    // to 8), four consecutive rows of a column per 16-byte store, only the
+    // row groups that hold a head; then lane l forms the outputs of
+    // d = l, l + 64, ... for every head (high + low row) and stores them
+    // coalesced along d
+    const int R = (2 * G + 7) & ~7;
+    float* sOT = (float*)smem;
 #pragma unroll
     for (int dt = 0; dt < NDT; dt++) {
 #pragma unroll
-        for (int vv = 0; vv < 16; vv++) {
-            const int r = 8 * (vv >> 2) + 4 * lg + (vv & 3);
-            if (PS || r < 2 * GC) sO[r * hd + 32 * dt + li] = acc[dt][vv];   // PS: rows >= GC are never read
+        for (int m4 = 0; m4 < 4; m4++) {
+            if (8 * m4 >= 2 * G) break;
+            *(f32x4a*)&sOT[(32 * dt + li) * R + 8 * m4 + 4 * lg] =
+                f32x4a{acc[dt][4 * m4], acc[dt][4 * m4 + 1], acc[dt][4 * m4 + 2], acc[dt][4 * m4 + 3]};
         }
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
-    if (MT && W > 1) {
-        // combine the W waves' states per column, waves in order:
-        // out = sum_w acc_w e^(m_w - M) / sum_w l_w e^(m_w - M), M = max_w m_w.
-        // The per-column quantities (wave weights, denominator, output row)
-        // are formed once per column; then each thread takes 8 consecutive d
-        // of a column: 16-byte LDS reads and one 16-byte store of 8 halves
-        // (the arithmetic per element as written above, in wave order, so the
-        // division and every rounding are those of the per-element form).
-        float* sML = (float*)(smem_wg + (size_t)W * wave_lds);     // [W][m[32] | l[32]]
-        float* sF = sML + W * 64;                                  // [W][32] wave weights
-        float* sDen = sF + ATTN_MAX_WAVES * 32;                    // [32] denominators
+    if (W > 1) {
+        // combine the W waves' states per head, waves in order:
+        // M = max_w m_w, num = sum_w acc_w e^(m_w - M), den = sum_w l_w e^(m_w - M);
+        // the workgroup's output (S == 1) or its partial (M, den, num).
+        // Wave weights e^(m_w - M) are formed once per (wave, head), then
+        // every thread issues all its LDS reads before it adds.
+        float* sML = (float*)(smem_wg + (size_t)W * wave_lds);     // [W][m[32] | l[32]], then f [W][32]
+        float* sF = sML + W * 64;
         if (lg == 0) { sML[wv * 64 + li] = run_m; sML[wv * 64 + 32 + li] = run_l; }
         __syncthreads();
         const int t = (int)threadIdx.x;
-        if (t < GC) {
+        if (t < W * G) {
+            const int u = t / G, h = t % G;
             float M = -FLT_MAX;
-            for (int u = 0; u < W; u++) M = fmaxf(M, sML[u * 64 + t]);
-            float den = 0.0f;
-            for (int u = 0; u < W; u++) {
-                const float f = expf(sML[u * 64 + t] - M);
-                sF[u * 32 + t] = f;
-                den += sML[u * 64 + 32 + t] * f;
-            }
-            sDen[t] = den;
+            for (int w = 0; w < W; w++) M = fmaxf(M, sML[w * 64 + h]);
+            sF[u * 32 + h] = expf(sML[u * 64 + h] - M);
+            if (u == 0) sF[ATTN_MAX_WAVES * 32 + h] = M;
         }
         __syncthreads();
-        const int nd8 = hd / 8;
-        const bool vec = ((uintptr_t)a.out & 15u) == 0;
-        for (int e = t; e < GC * nd8; e += 64 * W) {
-            const int c = e / nd8, d0 = (e - c * nd8) * 8;
-            float num[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-            for (int u = 0; u < W; u++) {
-                const float f = sF[u * 32 + c];
-                const float* so = (const float*)(smem_wg + (size_t)u * wave_lds);
-                const f32x4a h0 = *(const f32x4a*)&so[c * hd + d0], h1 = *(const f32x4a*)&so[c * hd + d0 + 4];
-                f32x4a l0 = f32x4a{0.0f, 0.0f, 0.0f, 0.0f}, l1 = l0;
-                if (!PS) { l0 = *(const f32x4a*)&so[(GC + c) * hd + d0]; l1 = *(const f32x4a*)&so[(GC + c) * hd + d0 + 4]; }
+        float* pm = a.part;
+        float* pl = a.part + (int64_t)a.n_heads * S;
+        float* pacc = a.part + (int64_t)a.n_heads * S * 2;
+        for (int e = t; e < G * hd; e += 64 * W) {
+            const int d = e / G, h = e % G;     // lanes: consecutive heads of one d, then d
+            float hi[ATTN_MAX_WAVES], lo[ATTN_MAX_WAVES], f[ATTN_MAX_WAVES], lv[ATTN_MAX_WAVES];
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    num[i] += (h0[i] + l0[i]) * f;
-                    num[4 + i] += (h1[i] + l1[i]) * f;
+            for (int u = 0; u < ATTN_MAX_WAVES; u++) {
+                if (u < W) {
+                    const float* so = (const float*)(smem_wg + (size_t)u * wave_lds);
+                    hi[u] = so[d * R + h];
+                    lo[u] = so[d * R + G + h];
+                    f[u] = sF[u * 32 + h];
+                    lv[u] = sML[u * 64 + 32 + h];
                 }
             }
-            const float den = sDen[c];
-            uint32_t o[4];
+            float num = 0.0f, den = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                o[i] = (uint32_t)f32_to_f16_bits(den > 0.0f ? num[2 * i] / den : 0.0f) |
-                       ((uint32_t)f32_to_f16_bits(den > 0.0f ? num[2 * i + 1] / den : 0.0f) << 16);
-            const int ct = c / G, ch = c - ct * G;
-            uint16_t* ot = a.out + (int64_t)(tok0 + ct) * a.n_heads * hd + (int64_t)(pbase + ch) * hd + d0;
-            if (vec) {
-                *(u32x4a*)ot = u32x4a{o[0], o[1], o[2], o[3]};
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; i++) { ot[2 * i] = (uint16_t)(o[i] & 0xFFFFu); ot[2 * i + 1] = (uint16_t)(o[i] >> 16); }
+            for (int u = 0; u < ATTN_MAX_WAVES; u++) {
+                if (u < W) {
+                    num += (hi[u] + lo[u]) * f[u];
+                    den += lv[u] * f[u];
+                }
             }
-            if (a.qcodes) {
-                // the 4 lanes of an aligned quad hold the 32 values of one
-                // quantiser block (hd % 32 == 0, nd8 % 4 == 0)
-                float v[8];
-#pragma unroll
-                for (int i = 0; i < 4; i++) { v[2 * i] = f16_bits_to_f32(o[i] & 0xFFFFu); v[2 * i + 1] = f16_bits_to_f32(o[i] >> 16); }
-                const int kb32 = ((pbase + ch) * hd + d0) >> 5, sub = (d0 >> 3) & 3;
-                if (a.q_i8) quant_chunk<true>(v, sub, kb32, tok0 + ct, a.q_npad, a.qcodes, a.qscl, true);
-                else        quant_chunk<false>(v, sub, kb32, tok0 + ct, a.q_npad, a.qcodes, a.qscl, false);
+            if (S == 1) {
+                a.out[(int64_t)(pbase + h) * hd + d] = f32_to_f16_bits(den > 0.0f ? num / den : 0.0f);
+            } else {
+                pacc[((int64_t)(pbase + h) * S + split) * hd + d] = num;
+                if (d == 0) {
+                    pm[(int64_t)(pbase + h) * S + split] = sF[ATTN_MAX_WAVES * 32 + h];
+                    pl[(int64_t)(pbase + h) * S + split] = den;
+                }
             }
         }
+#ifdef JLLM_ATTN_TRACE
+        AT_MARK(3);
+        {
+            const int gw = ((int)blockIdx.y * (int)gridDim.x + (int)blockIdx.x) * W + wv;
+            if (l < 4 && gw < 8192) {
+                uint64_t tv = 0;
+#pragma unroll
+                for (int i = 0; i < 4; i++) if (l == i) tv = tr[i];
+                g_attn_trace[gw * 4 + l] = tv;
+            }
+        }
+#endif
         return;
     }
     if (S == 1) {
         const float inv_l = run_l > 0.0f ? 1.0f / run_l : 0.0f;
-        for (int e = l; e < GC * hd; e += 64) {
-            const int c = e / hd, d = e % hd;
-            const float il = __shfl(inv_l, c, 64);
-            const int ct = MT ? c / G : 0, ch = MT ? c % G : c;
-            uint16_t* ot = a.out + (int64_t)(tok0 + ct) * a.n_heads * hd + (int64_t)(pbase + ch) * hd;
-            ot[d] = f32_to_f16_bits((PS ? sO[c * hd + d] : sO[c * hd + d] + sO[(GC + c) * hd + d]) * il);
+        for (int h = 0; h < G; h++) {
+            const float il = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv_l), h));
+            uint16_t* ot = a.out + (int64_t)(pbase + h) * hd;
+            for (int d = l; d < hd; d += 64)
+                ot[d] = f32_to_f16_bits((sOT[d * R + h] + sOT[d * R + G + h]) * il);
         }
         return;
     }
     float* pm = a.part;
     float* pl = a.part + (int64_t)a.n_heads * S;
-    float* pacc = a.part + (int64_t)a.n_heads * S * 2;
     if (li < G && lg == 0) {
         pm[(int64_t)(pbase + li) * S + split] = run_m;
         pl[(int64_t)(pbase + li) * S + split] = run_l;
     }
-    for (int e = l; e < G * hd; e += 64) {
-        const int h = e / hd, d = e % hd;
-        pacc[((int64_t)(pbase + h) * S + split) * hd + d] = sO[h * hd + d] + sO[(G + h) * hd + d];
+    float* pacc = a.part + (int64_t)a.n_heads * S * 2 + ((int64_t)pbase * S + split) * hd;
+    for (int h = 0; h < G; h++) {
+        for (int d = l; d < hd; d += 64) pacc[(int64_t)h * S * hd + d] = sOT[d * R + h] + sOT[d * R + G + h];
     }
+#ifdef JLLM_ATTN_TRACE
+    AT_MARK(3);
+    const int gw = blockIdx.y * gridDim.x + blockIdx.x;
+    if (l < 4 && gw < 8192) {
+        uint64_t tv = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) if (l == i) tv = tr[i];
+        g_attn_trace[gw * 4 + l] = tv;
+    }
+#endif
 }
 
 // out = sum_s acc_s e^(m_s - M) / sum_s l_s e^(m_s - M), M = max_s m_s
@@ -830,20 +635,15 @@ extern "C" int jllm_hip_attn_trace_read(uint64_t* host) {
 #endif
 
 hipError_t attn_launch(const AttnArgs& a, bool kv_int8, hipStream_t st) {
-    if (a.tokens < 1 || a.tq < 1 || (a.tokens > 1 && a.n_splits != 1) || (a.n_splits > 1 && a.tq != 1) ||
-        (a.n_heads / a.n_kv) * a.tq > (a.tq > 1 ? ATTN_MAX_COLUMNS : AT_MAXG))
-        return hipErrorInvalidValue;
-    dim3 grid(a.n_kv, a.n_splits, (a.tokens + a.tq - 1) / a.tq);
-    const bool mt = a.tq > 1;
+    if (a.tokens != 1 || a.n_heads / a.n_kv > AT_MAXG) return hipErrorInvalidValue;
+    dim3 grid(a.n_kv, a.n_splits);
     const int W = a.wsplit;
     if (W < 1 || W > ATTN_MAX_WAVES) return hipErrorInvalidValue;
-    if (a.qcodes && (!mt || W < 2 || a.head_dim % 32 || !a.qscl || a.q_npad < a.tokens)) return hipErrorInvalidValue;
-    const size_t lds = attn_lds_bytes(a.n_heads, a.n_kv, a.head_dim, a.tq, W);
-    const bool g4 = !mt && a.n_heads / a.n_kv <= 4;
+    const size_t lds = attn_lds_bytes(a.n_heads, a.n_kv, a.head_dim, W);
+    const bool g4 = a.n_heads / a.n_kv <= 4;
 #define ATTN_CASE(I8, HDV)                                                                                   \
-    if (mt)      hipLaunchKernelGGL((attn_partial_kernel<I8, HDV, true, false>), grid, dim3(64 * W), lds, st, a); \
-    else if (g4) hipLaunchKernelGGL((attn_partial_kernel<I8, HDV, false, true>), grid, dim3(64 * W), lds, st, a); \
-    else         hipLaunchKernelGGL((attn_partial_kernel<I8, HDV, false, false>), grid, dim3(64 * W), lds, st, a);
+    if (g4) hipLaunchKernelGGL((attn_partial_kernel<I8, HDV, true>), grid, dim3(64 * W), lds, st, a); \
+    else    hipLaunchKernelGGL((attn_partial_kernel<I8, HDV, false>), grid, dim3(64 * W), lds, st, a);
     switch (a.head_dim * 2 + (kv_int8 ? 1 : 0)) {
     case 64:  ATTN_CASE(false, 32) break;
     case 65:  ATTN_CASE(true, 32) break;

@@ -179,13 +179,10 @@ int prefill_attention(uint16_t* out, const uint16_t* q, const void* k, const voi
     a.counters = nullptr; a.part = nullptr;
     a.n_heads = n_heads; a.n_kv = n_kv_heads; a.head_dim = head_dim; a.cache_head_dim = cache_head_dim;
     a.seq = start_pos + 1; a.window = window; a.n_splits = 1; a.scale = scale; a.tokens = N;
-    // several query tokens per wave: each KV tile serves tq tokens x G heads
-    a.tq = ATTN_MAX_COLUMNS / (n_heads / n_kv_heads);
-    if (a.tq < 1) a.tq = 1;
-    a.wsplit = ATTN_PREFILL_WAVES;     // (used when tq > 1)
-    const bool q8 = quant && quantized && a.tq > 1 && a.wsplit > 1 && head_dim % 32 == 0;
+    a.tq = 1; a.wsplit = 1;
+    const bool q8 = quant && quantized && head_dim % 32 == 0;
     if (q8) { a.qcodes = quant->codes; a.qscl = quant->scl; a.q_npad = quant->npad; a.q_i8 = quant->i8 ? 1 : 0; }
-    const int st2 = launch_status(attn_launch(a, kv_int8 != 0, (hipStream_t)stream), "attention prefill");
+    const int st2 = launch_status(attn_prefill_launch(a, kv_int8 != 0, (hipStream_t)stream), "attention prefill");
     if (st2 == JLLM_OK && q8) *quantized = true;
     return st2;
 }

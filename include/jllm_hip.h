@@ -263,7 +263,7 @@ int jllm_hip_fp16_to_int8(int8_t* dst, float* scale_out, const uint16_t* src, in
  * (absolute position start_pos + t) attends to keys [0, start_pos + t] (the
  * last `window` of them when window > 0).  q and out are [N][n_heads x
  * head_dim]; cache layout and limits as jllm_hip_flash_attention_decode.
- * One wave per (KV head, token), no partials buffer.
+ * No partials buffer.
  * Replaces flash_attention_prefill_batched, jllm_kernels.h:354
  * (attention.cu:382-514, launcher :617-682). */
 int jllm_hip_flash_attention_prefill_batched(uint16_t* out, const uint16_t* q, const void* k, const void* v,

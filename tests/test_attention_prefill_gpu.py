@@ -1,0 +1,79 @@
+"""Prefill attention kernel forms against float64: every (columns, waves) form of
+the launcher at its edges -- partial last blocks and key tiles, KV heads with 1 to
+16 query heads, every head size, INT8 and FP16 caches, windows, padded cache
+heads -- and V scales beyond the fp16-safe bound of the lazily moved softmax
+reference.  Bar: the output is fp16 (one rounding, 2^-11 of the value) of fp32
+sums of ~22-bit probability products; 1e-3 of the largest output plus one fp16
+ulp of the value, the bar of the other attention tests."""
+import numpy as np
+import pytest
+import torch
+
+import jllm
+import synth
+from gpu_util import f16_to_f64, from_dev, print_case, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _want(q, k, v, start, window, scale):
+    """q [N, H, hd], k / v [ctx, KV, hd] in float64."""
+    N, H, hd = q.shape
+    ctx, KV = k.shape[0], k.shape[1]
+    pos, key = np.arange(start, start + N)[:, None], np.arange(ctx)[None, :]
+    dead = key > pos
+    if window:
+        dead |= key <= pos - window
+    out = np.empty_like(q)
+    for h in range(H):
+        g = h // (H // KV)
+        s = np.where(dead, -np.inf, q[:, h] @ k[:, g].T * scale)
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = (p / p.sum(1, keepdims=True)) @ v[:, g]
+    return out
+
+
+@pytest.mark.parametrize("H,KV,hd,pad,int8,N,start,window,vs_mul", [
+    (32, 8, 128, 0, True, 1, 0, 0, 1.0),            # one key
+    (32, 8, 128, 0, True, 7, 25, 0, 1.0),           # one partial block, keys end inside a tile
+    (32, 8, 128, 0, True, 256, 33, 0, 1.0),         # 256 blocks: 8 waves
+    (32, 8, 128, 0, True, 257, 0, 0, 1.0),          # 257 blocks: 4 waves
+    (32, 8, 128, 0, True, 300, 724, 0, 1.0),        # 1024 keys: 4 waves
+    (32, 8, 128, 0, True, 300, 725, 0, 1.0),        # 1025 keys: 64 columns
+    (32, 8, 128, 0, False, 261, 800, 0, 1.0),       # the same form, fp16 cache
+    (32, 8, 128, 0, True, 263, 900, 100, 1.0),      # window: short key ranges
+    (32, 8, 128, 0, True, 261, 1200, 1100, 1.0),    # window: long key ranges
+    (32, 8, 128, 0, True, 40, 100, 0, 3e4),         # V scales beyond AP_VS_MAX (values near the fp16 limit)
+    (8, 8, 64, 0, True, 70, 11, 0, 1.0),
+    (12, 4, 96, 0, True, 50, 60, 0, 1.0),           # 3 heads per KV head: 30 of 32 columns live
+    (12, 4, 96, 0, False, 50, 60, 20, 1.0),
+    (32, 2, 32, 0, True, 9, 40, 0, 1.0),            # 16 heads per KV head: 2 tokens a block
+    (8, 2, 32, 0, False, 33, 31, 0, 1.0),
+    (16, 2, 128, 32, True, 20, 50, 0, 1.0),         # cache heads wider than the head
+    (8, 2, 64, 0, False, 64, 64, 0, 1.0),
+])
+def test_prefill_attention_forms(dev, H, KV, hd, pad, int8, N, start, window, vs_mul):
+    print_case("attn_prefill_form", H, KV, hd, pad, int8, N, start, window, vs_mul)
+    g = synth.rng(H * 1000 + hd + N + start)
+    ctx, chd, scale = start + N, hd + pad, 1.0 / np.sqrt(hd)
+    q = synth.x_f16(g, (N, H, hd))
+    out = torch.empty(N * H * hd, dtype=torch.int16, device=dev)
+    if int8:
+        k, v = synth.kv_int8(g, ctx, KV, chd), synth.kv_int8(g, ctx, KV, chd)
+        ks, vs = synth.kv_scales(g, ctx, KV), synth.kv_scales(g, ctx, KV) * np.float32(vs_mul)
+        vs = np.minimum(vs, np.float32(500.0)) if vs_mul == 1.0 else np.minimum(vs, np.float32(4000.0))
+        if vs_mul != 1.0:
+            v = np.clip(v, -12, 12)                  # |v * vs| <= 48000 stays an fp16 number
+        args = [to_dev(k), to_dev(v), to_dev(ks), to_dev(vs)]
+        kf, vf = k[..., :hd] * ks[..., None].astype(np.float64), v[..., :hd] * vs[..., None].astype(np.float64)
+    else:
+        kh = (g.standard_normal((ctx, KV, chd)) * 0.5).astype(np.float16)
+        vh = g.standard_normal((ctx, KV, chd)).astype(np.float16)
+        args = [to_dev(kh.view(np.uint16)), to_dev(vh.view(np.uint16)), None, None]
+        kf, vf = kh[..., :hd].astype(np.float64), vh[..., :hd].astype(np.float64)
+    jllm.call("jllm_hip_flash_attention_prefill_batched", out, to_dev(q), args[0], args[1], H, KV, hd, chd, N, start,
+              scale, int(int8), args[2], args[3], window)
+    got = f16_to_f64(from_dev(out, np.uint16)).reshape(N, H, hd)
+    want = _want(f16_to_f64(q).reshape(N, H, hd), kf, vf, start, window, scale)
+    err = np.abs(got - want)
+    assert np.all(err <= 1e-3 * np.abs(want).max() + np.abs(want) * 2 ** -10), float(err.max())
