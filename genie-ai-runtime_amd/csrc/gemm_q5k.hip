@@ -34,6 +34,7 @@
 // does not change the sum.
 #include "kq_common.h"
 #include "mmq.h"
+#include "mmq_tile.h"
 
 namespace jllm_hip {
 namespace {
@@ -44,7 +45,7 @@ typedef _Float16 h8q __attribute__((ext_vector_type(8)));
 typedef float f32x16q __attribute__((ext_vector_type(16)));
 typedef float f32x4q __attribute__((ext_vector_type(4)));
 
-constexpr int TM = 128, TN = 64, THREADS = 256;
+constexpr int TM = 128, TN = 64, THREADS = MMQ_TILE_THREADS;
 constexpr int XS = QK_K + 8;          // fp16 per staged token row (16 B pad against bank conflicts)
 
 // 8 code bytes (values 0..31) -> 8 fp16 values times the sub-block scale:
@@ -230,18 +231,14 @@ void gemm_q5k_kernel(void* __restrict__ y, const uint8_t* __restrict__ W, const 
         __syncthreads();
     }
 
+    // the output tile through the activation tile's LDS (the last super-block's
+    // barrier has passed)
+    static_assert(mmq_tile_bytes<OUT == 1>(TN) <= sizeof(sX), "output tile exceeds the LDS");
+    uint8_t* T = (uint8_t*)sX;
 #pragma unroll
-    for (int tt = 0; tt < 2; tt++) {
-        const int tok = col0 + 32 * tt + li;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = row0 + 32 * w + 8 * (v >> 2) + 4 * kg + (v & 3);
-            if (r < M && tok < N) {
-                if (OUT == 1) ((float*)y)[(int64_t)blockIdx.y * N * M + (int64_t)tok * M + r] = acc[tt][v];
-                else          ((uint16_t*)y)[(int64_t)tok * M + r] = f32_to_f16_bits(acc[tt][v]);
-            }
-        }
-    }
+    for (int tt = 0; tt < 2; tt++) mmq_put_tile<OUT == 1>(T, 32 * tt + li, 32 * w + 4 * kg, acc[tt]);
+    __syncthreads();
+    mmq_store_tile<OUT == 1>(y, T, row0, col0, TN, M, N);
 }
 
 }  // namespace

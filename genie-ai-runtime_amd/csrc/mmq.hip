@@ -39,6 +39,7 @@
 #include "mmq.h"
 #include "qk_front.h"
 #include "quant_chunk.h"
+#include "mmq_tile.h"
 #include <algorithm>
 #include <stdlib.h>
 
@@ -53,7 +54,7 @@ typedef _Float16 h8m __attribute__((ext_vector_type(8)));
 typedef _Float16 h4m __attribute__((ext_vector_type(4)));
 typedef float f32x16m __attribute__((ext_vector_type(16)));
 
-constexpr int MMQ_THREADS = 256;
+constexpr int MMQ_THREADS = MMQ_TILE_THREADS;
 constexpr int TM = 128;                 // rows per workgroup tile (4 waves x 32)
 constexpr int TN = MMQ_TILE_N;          // tokens per workgroup tile (64)
 
@@ -669,18 +670,14 @@ __device__ __forceinline__ void mmq_q4k_body(const MmqSegs& sg, const uint8_t* _
         }
         return;
     }
+    // the output tile through the ring's LDS
+    __builtin_amdgcn_s_waitcnt(0);                     // the ring's last DMA has landed
+    static_assert(mmq_tile_bytes<OUT == 1>(TNv) <= sizeof(smem), "output tile exceeds the LDS ring");
+    __syncthreads();
 #pragma unroll
-    for (int tt = 0; tt < TT; tt++) {
-        const int tok = col0 + 32 * tt + li;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = row0 + 32 * w + 8 * (v >> 2) + 4 * g + (v & 3);
-            if (r < M && tok < N) {
-                if (OUT == 1) ((float*)y)[(int64_t)blockIdx.y * N * M + (int64_t)tok * M + r] = acc[tt][v];
-                else          ((uint16_t*)y)[(int64_t)tok * M + r] = f32_to_f16_bits(acc[tt][v]);
-            }
-        }
-    }
+    for (int tt = 0; tt < TT; tt++) mmq_put_tile<OUT == 1>(smem, 32 * tt + li, 32 * w + 4 * g, acc[tt]);
+    __syncthreads();
+    mmq_store_tile<OUT == 1>(y, smem, row0, col0, TNv, M, N);
 }
 
 template <int OUT, int TT>
@@ -950,18 +947,14 @@ void mmq_q6k_kernel(void* __restrict__ y, const uint8_t* __restrict__ W, const u
         hd0 = hd1;
     }
     if (OUT == 2) return;
+    // the output tile through LDS (the last stage's DMA has been waited for)
+    __builtin_amdgcn_s_waitcnt(0);
+    static_assert(mmq_tile_bytes<OUT == 1>(Q6_TN) <= sizeof(smem), "output tile exceeds the LDS ring");
+    __syncthreads();
 #pragma unroll
-    for (int tt = 0; tt < 4; tt++) {
-        const int tok = col0 + 32 * tt + li;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = row0 + 32 * w + 8 * (v >> 2) + 4 * g + (v & 3);
-            if (r < M && tok < N) {
-                if (OUT == 1) ((float*)y)[(int64_t)blockIdx.y * N * M + (int64_t)tok * M + r] = acc[tt][v];
-                else          ((uint16_t*)y)[(int64_t)tok * M + r] = f32_to_f16_bits(acc[tt][v]);
-            }
-        }
-    }
+    for (int tt = 0; tt < 4; tt++) mmq_put_tile<OUT == 1>(smem, 32 * tt + li, 32 * w + 4 * g, acc[tt]);
+    __syncthreads();
+    mmq_store_tile<OUT == 1>(y, smem, row0, col0, Q6_TN, M, N);
 }
 
 hipError_t mmq_launch(void* y, const uint8_t* W, int type, const void* codes, const uint32_t* scl, int M, int N,
