@@ -83,28 +83,41 @@ __device__ __forceinline__ void load_a(ARegs& a, const uint8_t* blk, int kg) {
     for (int il = 0; il < 4; il++) a.qs[il] = *(const u32x4q*)(blk + 48 + 32 * il + 16 * kg);
 }
 
-// The thread's share of the activation tile: token t >> 2, fp16 values
-// [64 q, 64 q + 64) of the super-block (q = t & 3).
+// The thread's share of the activation tile: token t >> 2, of each sub-block
+// j the fp16 values [8 q, 8 q + 8) (q = t & 3): a load instruction of four
+// lanes covers 64 contiguous bytes of a row (with 128 contiguous bytes per
+// thread every instruction touched 64 separate lines, each line in eight
+// instructions: 9728 x 2560 at 300 tokens 43.5 us against 38.3 us).  The sums
+// X_j then come from four lanes of eight values each instead of one chain of
+// 32: fp32 as before, a shorter chain.
 struct XRegs { u32x4q v[8]; };
 
 __device__ __forceinline__ void load_x(XRegs& r, const uint16_t* src) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) r.v[i] = *(const u32x4q*)(src + 8 * i);
+    for (int j = 0; j < 8; j++) r.v[j] = *(const u32x4q*)(src + 32 * j);
 }
 
-// Store the thread's 64 values and the two sub-block sums (X/32 as fp16 hi + lo).
+// a + the value of the lane whose index differs by the quad permutation P
+template <int P> __device__ __forceinline__ float quad_add(float a) {
+    return a + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, a), P, 0xF, 0xF, true));
+}
+
+// Store the thread's 64 values and, of the eight sub-block sums that the
+// token's four lanes add up, its two (X/32 as fp16 hi + lo).
 __device__ __forceinline__ void commit_x(const XRegs& r, uint16_t* sx, uint16_t* ss, int tok, int q) {
-    uint16_t* dst = sx + tok * XS + 64 * q;
-#pragma unroll
-    for (int i = 0; i < 8; i++) *(u32x4q*)(dst + 8 * i) = r.v[i];
+    uint16_t* dst = sx + tok * XS + 8 * q;
     const uint32_t one = 0x3C003C00u;
     float s[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        float t = s[i >> 2];
-        t = fdot2(r.v[i].x, one, t); t = fdot2(r.v[i].y, one, t);
-        t = fdot2(r.v[i].z, one, t); t = fdot2(r.v[i].w, one, t);
-        s[i >> 2] = t;
+    for (int j = 0; j < 8; j++) {
+        *(u32x4q*)(dst + 32 * j) = r.v[j];
+        float t = fdot2(r.v[j].x, one, 0.0f);
+        t = fdot2(r.v[j].y, one, t);
+        t = fdot2(r.v[j].z, one, t);
+        t = fdot2(r.v[j].w, one, t);
+        t = quad_add<0xB1>(t);
+        t = quad_add<0x4E>(t);
+        if ((j >> 1) == q) s[j & 1] = t;
     }
     uint32_t hi = 0, lo = 0;
 #pragma unroll
@@ -142,7 +155,7 @@ void gemm_q5k_kernel(void* __restrict__ y, const uint8_t* __restrict__ W, const 
 
     const uint8_t* wrow = W + (int64_t)min(row0 + 32 * w + li, M - 1) * nb * Q5K_BYTES;   // rows past M re-read the last
     const int xtok = t >> 2, xq = t & 3;
-    const uint16_t* xsrc = x + (int64_t)min(col0 + xtok, N - 1) * K + 64 * xq;            // tokens past N: the last
+    const uint16_t* xsrc = x + (int64_t)min(col0 + xtok, N - 1) * K + 8 * xq;            // tokens past N: the last
 
     f32x16q acc[2];
 #pragma unroll
