@@ -201,11 +201,16 @@ void attn_prefill_kernel(AttnArgs a) {
     const int x16 = 16 * ap_swz<NP>(li);
     int kx = SW ? ((8 * NP * lg) ^ x16) : 8 * NP * lg, vx = SW ? ((16 * lg) ^ x16) : 16 * lg;
     auto off = [&](int x, int c) { return li * NP * 16 + (SW ? (x ^ (16 * c)) : x + 16 * c); };
-    // one scale per lane: ks of key li (lg = 0), vs of key li (lg = 1)
-    const float* sp = lg ? a.vs : a.ks;
+    // one scale per lane: ks of key li (lg = 0), vs of key li (lg = 1); 1 where the
+    // caller has none.  Such a lane loads as well (the first word of q, unused):
+    // the waits below count the wave's loads, so every INT8 call issues exactly
+    // one scale load per tile.
+    const bool own_sc = (lg ? a.vs : a.ks) != nullptr;
+    const float* sp = own_sc ? (lg ? a.vs : a.ks) + kvh : (const float*)a.q;
+    const int sc_row = own_sc ? a.n_kv : 0;
     float scn = 1.0f;
     auto load_sc = [&](int p0) {
-        if (INT8 && sp) scn = sp[(int64_t)min(p0 + li, seq - 1) * a.n_kv + kvh];
+        if (INT8) scn = sp[(int64_t)min(p0 + li, seq - 1) * sc_row];
     };
     const int first = lo_pos + wv * AT_KEYS;
     constexpr int stride = W * AT_KEYS;
@@ -243,10 +248,11 @@ void attn_prefill_kernel(AttnArgs a) {
         // (opaque per tile: the addresses formed from these few lane constants
         // would otherwise be hoisted and spilled)
         asm volatile("" : "+v"(kx), "+v"(vx), "+v"(lane));
+        const float scv = own_sc ? scn : 1.0f;
         // per-key scales through LDS to the lanes that hold a key's scores
         // (keys 8m + 4lg + [0,4))
-        if (INT8) sS[32 * lg + li] = lg ? scn : scn * (a.scale * LOG2E);
-        const float slack = __builtin_amdgcn_ballot_w64(INT8 && lg && !(fabsf(scn) <= AP_VS_MAX)) == 0 ? AP_SLACK : 0.0f;
+        if (INT8) sS[32 * lg + li] = lg ? scv : scv * (a.scale * LOG2E);
+        const float slack = __builtin_amdgcn_ballot_w64(INT8 && lg && !(fabsf(scv) <= AP_VS_MAX)) == 0 ? AP_SLACK : 0.0f;
         // 1. transposed scores
         ap_wait_vm<NI>();                                // the K rows (the V rows may be in flight)
         // All K pieces first, the q pieces two steps ahead of their products,

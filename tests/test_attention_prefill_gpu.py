@@ -77,3 +77,31 @@ def test_prefill_attention_forms(dev, H, KV, hd, pad, int8, N, start, window, vs
     want = _want(f16_to_f64(q).reshape(N, H, hd), kf, vf, start, window, scale)
     err = np.abs(got - want)
     assert np.all(err <= 1e-3 * np.abs(want).max() + np.abs(want) * 2 ** -10), float(err.max())
+
+
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("N,start", [(20, 700), (300, 200), (300, 900)])    # 8 waves, 4 waves, 64 columns
+@pytest.mark.parametrize("with_ks,with_vs", [(False, False), (True, False), (False, True)])
+def test_prefill_attention_without_scales(dev, hd, N, start, with_ks, with_vs):
+    """INT8 caches whose k_scales and / or v_scales are NULL (= 1.0), several key
+    tiles per wave: the kernel's waits count its loads, so a call without scale
+    pointers has to issue as many as one with them."""
+    print_case("attn_prefill_no_scales", hd, N, start, with_ks, with_vs)
+    H, KV = 32, 8
+    g = synth.rng(hd + N + start)
+    ctx = start + N
+    q = synth.x_f16(g, (N, H, hd))
+    # without scales K codes of -1, 0, 1: scores of order 1, so that every key counts
+    k = synth.kv_int8(g, ctx, KV, hd) if with_ks else g.integers(-1, 2, size=(ctx, KV, hd), dtype=np.int8)
+    v = synth.kv_int8(g, ctx, KV, hd)
+    ks, vs = synth.kv_scales(g, ctx, KV), synth.kv_scales(g, ctx, KV)
+    scale = 1.0 / np.sqrt(hd)
+    out = torch.empty(N * H * hd, dtype=torch.int16, device=dev)
+    jllm.call("jllm_hip_flash_attention_prefill_batched", out, to_dev(q), to_dev(k), to_dev(v), H, KV, hd, hd, N, start,
+              scale, 1, to_dev(ks) if with_ks else None, to_dev(vs) if with_vs else None, 0)
+    got = f16_to_f64(from_dev(out, np.uint16)).reshape(N, H, hd)
+    kf = k.astype(np.float64) * (ks[..., None].astype(np.float64) if with_ks else 1.0)
+    vf = v.astype(np.float64) * (vs[..., None].astype(np.float64) if with_vs else 1.0)
+    want = _want(f16_to_f64(q).reshape(N, H, hd), kf, vf, start, 0, scale)
+    err = np.abs(got - want)
+    assert np.all(err <= 1e-3 * np.abs(want).max() + np.abs(want) * 2 ** -10), float(err.max())
