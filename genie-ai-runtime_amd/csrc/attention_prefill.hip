@@ -16,10 +16,13 @@ namespace jllm_hip {
 // One workgroup of W waves per (KV head, block of tq tokens).  Its columns
 // are the (token, head) pairs of the block -- column c = token tok0 + c / G,
 // head kvh * G + c % G -- in NG groups of 32, and every wave holds all of
-// them; the waves deal the 32-key tiles among themselves (tile t to wave
-// t % W, by absolute position, so a column's result does not depend on
-// how a prompt is cut into chunks) and their softmax states are combined in
-// LDS in wave order.
+// them.  The 32-key tiles are dealt to AP_STATES = 8 softmax states, tile t to
+// state t % 8, which are combined in LDS in a fixed order: 8 waves hold one
+// each; of 4 waves each forms two, one after the other (wave w state w, then
+// w + 4).  So every form of the launch gives the same bits, and with them a
+// token's result does not depend on how a prompt is cut into calls, as long as
+// its window does not bind (where it does, the tiles start at the window start
+// of the block's first token).
 //
 // Everything a tile needs after its loads stays in a wave's registers.  Lane
 // (li = lane & 31, lg = lane >> 5), MFMA elements v = 0..15 <-> index
@@ -42,9 +45,11 @@ namespace jllm_hip {
 // exponentials 9), and a 32-key x 64-column tile takes ~430 of them against
 // 1664 clocks of MFMA; hence the one-operation conversions below, the scores
 // formed relative to the reference (one fma), and two column groups per K / V
-// conversion.  32 / 8 heads x 128, INT8 KV, 512 tokens: at start 0 17.1 -> 11.6
-// us, at start 7680 165 -> 114 us (584 TFLOP/s of q.k and p.v products) against
+// conversion.  32 / 8 heads x 128, INT8 KV, 512 tokens: at start 0 17.1 -> 12.8
+// us, at start 7680 166 -> 113 us (584 TFLOP/s of q.k and p.v products) against
 // the form it replaces (P' through LDS, lane-per-row loads, exact maxima).
+// The second state of a wave costs the 4-wave form 0.9-1.1 us a call (11.7 us at
+// start 0 with one state per wave, whose bits followed the form).
 //
 // A column's softmax reference is not its running maximum but a value at most
 // AP_SLACK (in base 2) below it, so that the accumulators are rescaled only
@@ -54,6 +59,7 @@ namespace jllm_hip {
 // the fp16 range times 1/127) take the exact maximum.
 constexpr float AP_SLACK = 6.0f, AP_VS_MAX = 1000.0f;
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr int AP_STATES = 8;
 
 typedef __attribute__((address_space(3))) void ap_lds_void;
 
@@ -139,9 +145,11 @@ void attn_prefill_kernel(AttnArgs a) {
     constexpr int Q_B = 32 * NG * QLD * 2, LOOP_B = Q_B + W * (2 * TILE_B + 256);
     constexpr int COMB_B = W * 32 * OLD * 4;
     constexpr int AREA_B = LOOP_B > COMB_B ? LOOP_B : COMB_B;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[AREA_B + (W * 2 + 1) * NG * 32 * 4];
-    float (*sML)[NG][2][32] = (float (*)[NG][2][32])(smem + AREA_B);    // [wave]: m, l of its columns
-    float (*sDen)[32] = (float (*)[32])(smem + AREA_B + W * 2 * NG * 32 * 4);
+    __shared__ __attribute__((aligned(16))) uint8_t smem[AREA_B + (AP_STATES * 2 + 1) * NG * 32 * 4];
+    float (*sML)[NG][2][32] = (float (*)[NG][2][32])(smem + AREA_B);    // [state]: m, l of the columns
+    float (*sDen)[32] = (float (*)[32])(smem + AREA_B + AP_STATES * 2 * NG * 32 * 4);
+    constexpr bool TWO = W < AP_STATES;                 // a wave forms two states
+    static_assert(W == AP_STATES || 2 * W == AP_STATES, "states per wave");
 
     const int t = (int)threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -213,7 +221,7 @@ void attn_prefill_kernel(AttnArgs a) {
         if (INT8) scn = sp[(int64_t)min(p0 + li, seq - 1) * sc_row];
     };
     const int first = lo_pos + wv * AT_KEYS;
-    constexpr int stride = W * AT_KEYS;
+    constexpr int stride = AP_STATES * AT_KEYS;
     if (first < seq) { load_rows(a.k, sK, first, l); load_sc(first); load_rows(a.v, sV, first, l); }
 
     // the columns' q rows, shared by the waves (zeros past the live columns)
@@ -239,12 +247,27 @@ void attn_prefill_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < NDT; i++) acc[g][i] = f32x16{};
     }
+    // TWO: the wave's first state, once its second one has begun (until then: no keys)
+    bool second = false;
+    float m1[NG], l1[NG];
+    f32x16 acc1[NG][TWO ? NDT : 1];
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        m1[g] = -FLT_MAX;
+        l1[g] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < (TWO ? NDT : 1); i++) acc1[g][i] = f32x16{};
+    }
     __syncthreads();
 
     int lane = l;
 #pragma unroll 1
-    for (int p0 = first; p0 < seq; p0 += stride) {
-        const int n = min(AT_KEYS, seq - p0), pn = min(p0 + stride, seq - 1);
+    for (int p0 = first; p0 < seq;) {
+        // the wave's next tile (the first of its second state after the last of its first)
+        int next = p0 + stride;
+        const bool turn2 = TWO && !second && next >= seq;
+        if (turn2) next = first + W * AT_KEYS;
+        const int n = min(AT_KEYS, seq - p0), pn = min(next, seq - 1);
         // (opaque per tile: the addresses formed from these few lane constants
         // would otherwise be hoisted and spilled)
         asm volatile("" : "+v"(kx), "+v"(vx), "+v"(lane));
@@ -252,7 +275,7 @@ void attn_prefill_kernel(AttnArgs a) {
         // per-key scales through LDS to the lanes that hold a key's scores
         // (keys 8m + 4lg + [0,4))
         if (INT8) sS[32 * lg + li] = lg ? scv : scv * (a.scale * LOG2E);
-        const float slack = __builtin_amdgcn_ballot_w64(INT8 && lg && !(fabsf(scv) <= AP_VS_MAX)) == 0 ? AP_SLACK : 0.0f;
+        const uint32_t big_vs = INT8 ? (uint32_t)(__builtin_amdgcn_ballot_w64(lg && !(fabsf(scv) <= AP_VS_MAX)) >> 32) : 0u;
         // 1. transposed scores
         ap_wait_vm<NI>();                                // the K rows (the V rows may be in flight)
         // All K pieces first, the q pieces two steps ahead of their products,
@@ -324,8 +347,15 @@ void attn_prefill_kernel(AttnArgs a) {
         }
         // 2. online softmax of the lane's column(s).  A column's reference moves
         // only when its maximum passes it by more than `slack`; its first live
-        // key sets it.
-        float up[NG];
+        // key sets it.  (Keys past the column's causal bound have no say.)
+        float slack[NG], up[NG];
+#pragma unroll
+        for (int g = 0; g < NG; g++) slack[g] = AP_SLACK;
+        if (big_vs) {
+#pragma unroll
+            for (int g = 0; g < NG; g++)
+                if (seq_c[g] > p0 && (big_vs << max(0, AT_KEYS - (seq_c[g] - p0))) != 0) slack[g] = 0.0f;
+        }
         bool mv[NG], moved = false;
 #pragma unroll
         for (int g = 0; g < NG; g++) {
@@ -335,7 +365,7 @@ void attn_prefill_kernel(AttnArgs a) {
             float a0, a1;
             wave_halves(mx, a0, a1);
             mx = fmaxf(a0, a1);
-            mv[g] = mx > none[g] + slack;
+            mv[g] = mx > none[g] + slack[g];
             up[g] = mv[g] ? mx : 0.0f;
             moved |= mv[g];
         }
@@ -410,16 +440,36 @@ void attn_prefill_kernel(AttnArgs a) {
         }
         ap_wait_lds();                                   // the V rows have been read
         load_rows(a.v, sV, pn, lane);
+        p0 = next;
+        if (TWO && turn2 && next < seq) {
+            second = true;
+#pragma unroll
+            for (int g = 0; g < NG; g++) {
+                m1[g] = none[g] == 0.0f ? run_m[g] : -FLT_MAX;
+                l1[g] = run_l[g];
+                run_m[g] = 0.0f;
+                none[g] = -FLT_MAX;
+                run_l[g] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < (TWO ? NDT : 1); i++) { acc1[g][i] = acc[g][i]; acc[g][i] = f32x16{}; }
+            }
+        }
     }
     ap_wait_vm<0>();                                     // the rows fetched past the last tile have landed
 
-    // 5. the waves' states combined per column, waves in order:
-    // out = sum_w acc_w 2^(m_w - M) / sum_w l_w 2^(m_w - M), M = max_w m_w
+    // 5. the states combined per column:
+    // out = sum_u acc_u 2^(m_u - M) / sum_u l_u 2^(m_u - M), M = max_u m_u; the
+    // numerator as the sum over w < 4 of the sums of states w and w + 4
     if (lg == 0) {
 #pragma unroll
         for (int g = 0; g < NG; g++) {
-            sML[wv][g][0][li] = none[g] == 0.0f ? run_m[g] : -FLT_MAX;
-            sML[wv][g][1][li] = run_l[g];
+            const int u = TWO && second ? wv + W : wv;
+            sML[u][g][0][li] = none[g] == 0.0f ? run_m[g] : -FLT_MAX;
+            sML[u][g][1][li] = run_l[g];
+            if (TWO) {
+                sML[wv + W - (u - wv)][g][0][li] = m1[g];
+                sML[wv + W - (u - wv)][g][1][li] = l1[g];
+            }
         }
     }
     __syncthreads();                                     // (every wave has read its last q rows, too)
@@ -430,20 +480,29 @@ void attn_prefill_kernel(AttnArgs a) {
     for (int g = 0; g < NG; g++) {
         float M = sML[0][g][0][li];
 #pragma unroll
-        for (int u = 1; u < W; u++) M = fmaxf(M, sML[u][g][0][li]);
-        const float f = __builtin_amdgcn_exp2f(sML[wv][g][0][li] - M);
+        for (int u = 1; u < AP_STATES; u++) M = fmaxf(M, sML[u][g][0][li]);
+        const float f = __builtin_amdgcn_exp2f((none[g] == 0.0f ? run_m[g] : -FLT_MAX) - M);
+        const float f1 = TWO ? __builtin_amdgcn_exp2f(m1[g] - M) : 0.0f;
         if (wv == 0 && lg == 0) {
             float den = 0.0f;
 #pragma unroll
-            for (int u = 0; u < W; u++) den += sML[u][g][1][li] * __builtin_amdgcn_exp2f(sML[u][g][0][li] - M);
+            for (int u = 0; u < AP_STATES; u++) den += sML[u][g][1][li] * __builtin_amdgcn_exp2f(sML[u][g][0][li] - M);
             sDen[g][li] = den;
         }
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
-            for (int m4 = 0; m4 < 4; m4++)
-                *(f32x4a*)&sO[(wv * 32 + li) * OLD + 32 * dt + 8 * m4 + 4 * lg] =
-                    f32x4a{acc[g][dt][4 * m4] * f, acc[g][dt][4 * m4 + 1] * f, acc[g][dt][4 * m4 + 2] * f, acc[g][dt][4 * m4 + 3] * f};
+            for (int m4 = 0; m4 < 4; m4++) {
+                // (products and sum rounded one by one, as where two waves hold the states)
+#pragma clang fp contract(off)
+                f32x4a o;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    o[i] = acc[g][dt][4 * m4 + i] * f;
+                    if (TWO) o[i] += acc1[g][TWO ? dt : 0][4 * m4 + i] * f1;
+                }
+                *(f32x4a*)&sO[(wv * 32 + li) * OLD + 32 * dt + 8 * m4 + 4 * lg] = o;
+            }
         __syncthreads();
         // each thread: 8 consecutive d of a column
         const int gc = min(32, GC - 32 * g);
@@ -451,8 +510,12 @@ void attn_prefill_kernel(AttnArgs a) {
             const int cl = e / nd8, d0 = (e - cl * nd8) * 8, c = 32 * g + cl;
             f32x4a n0 = f32x4a{0.0f, 0.0f, 0.0f, 0.0f}, n1 = n0;
 #pragma unroll
-            for (int u = 0; u < W; u++) {
-                const f32x4a h0 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0], h1 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0 + 4];
+            for (int u = 0; u < AP_STATES / 2; u++) {
+                f32x4a h0 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0], h1 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0 + 4];
+                if (!TWO) {
+                    h0 += *(const f32x4a*)&sO[((u + AP_STATES / 2) * 32 + cl) * OLD + d0];
+                    h1 += *(const f32x4a*)&sO[((u + AP_STATES / 2) * 32 + cl) * OLD + d0 + 4];
+                }
 #pragma unroll
                 for (int i = 0; i < 4; i++) { n0[i] += h0[i]; n1[i] += h1[i]; }
             }
@@ -489,14 +552,18 @@ void attn_prefill_kernel(AttnArgs a) {
 }
 
 // Column groups and waves of a workgroup, by the grid and the keys a block
-// sees (32 / 8 heads x 128, INT8 KV, us for 32 columns x 4 waves / 32 x 8 /
-// 64 x 8; N tokens at start):
+// sees; the results do not depend on it (32 / 8 heads x 128, INT8 KV, us for 32
+// columns x 4 waves / 32 x 8 / 64 x 8; N tokens at start):
 //   a grid of 32-column blocks that leaves CUs idle: 8 waves share a block's
-//   keys (N = 32 at 1000: 17.2 / 12.9 / 19.2; 128 at 4000: 51.1 / 36.9 / 55.1);
-//   short key ranges: 4 waves, so that the combination of the waves' states
-//   stays small (512 at 0: 12.2 / 15.0 / 13.9; 512 at 512: 21.0 / 22.7 / 20.6);
+//   keys, however few (N = 33 at 0: 6.8 / 6.3 / 9.5; 32 at 1000: 18.1 / 13.0 /
+//   19.9; 128 at 4000: 50.5 / 36.1 / 54.4);
+//   short key ranges: 4 waves, two workgroups on a CU (512 at 0: 12.8 / 14.9 /
+//   14.3; 512 at 256: 16.5 / 18.7 / 17.4; 512 at 512: 20.9 / 22.4 / 20.8);
 //   else 64 columns, half the K / V conversions and reads per column (512 at
-//   1024: 29.3 / 30.3 / 27.0; 512 at 7680: 140 / 143 / 115).
+//   1024: 29.4 / 30.1 / 27.6; 512 at 7680: 139 / 140 / 114).
+// FP16 caches, head sizes 32 to 96, 1 to 16 heads on each of 1 to 32 KV heads and
+// windows (some 80 calls in all) take a form within 7 % of their best one, except 512
+// tokens at 2000 with a window of 512 (17.6 / 19.5 / 15.8).
 enum { AP_1x4, AP_1x8, AP_2x8 };
 static int attn_prefill_form(const AttnArgs& a) {
     const int tq1 = ATTN_MAX_COLUMNS / (a.n_heads / a.n_kv);

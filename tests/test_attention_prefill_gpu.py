@@ -105,3 +105,46 @@ def test_prefill_attention_without_scales(dev, hd, N, start, with_ks, with_vs):
     want = _want(f16_to_f64(q).reshape(N, H, hd), kf, vf, start, 0, scale)
     err = np.abs(got - want)
     assert np.all(err <= 1e-3 * np.abs(want).max() + np.abs(want) * 2 ** -10), float(err.max())
+
+
+@pytest.mark.parametrize("H,KV,hd,int8,big_vs", [
+    (32, 8, 128, True, False),
+    (32, 8, 128, True, True),           # single V scales beyond AP_VS_MAX
+    (32, 8, 128, False, False),
+    (12, 4, 96, True, False),           # blocks of 10 and 21 tokens
+    (8, 2, 64, True, False),
+    (32, 32, 32, False, False),
+])
+def test_prefill_attention_bits_do_not_depend_on_the_cut(dev, H, KV, hd, int8, big_vs):
+    """A prompt of 1300 tokens in one call and cut into calls that take every form
+    of the launcher at every key range: the same bits, whichever form a token's
+    call takes."""
+    print_case("attn_prefill_cut", H, KV, hd, int8, big_vs)
+    g = synth.rng(H + hd)
+    T = 1300
+    q = to_dev(synth.x_f16(g, (T, H, hd)))
+    ks = vs = None
+    if int8:
+        k, v = synth.kv_int8(g, T, KV, hd), synth.kv_int8(g, T, KV, hd)
+        ks, vs = synth.kv_scales(g, T, KV), synth.kv_scales(g, T, KV)
+        if big_vs:
+            vs[::37] = 2000.0
+            v = np.clip(v, -12, 12)
+        ks, vs = to_dev(ks), to_dev(vs)
+    else:
+        k, v = (g.standard_normal((T, KV, hd)).astype(np.float16).view(np.uint16) for _ in range(2))
+    k, v = to_dev(k), to_dev(v)
+    q = q.view(T, H * hd)
+    want = None
+    for cut in ([1300], [512, 512, 276], [256] * 5 + [20], [100] * 13, [505, 795], [509, 30, 761], [511, 1, 700, 88]):
+        out = torch.zeros_like(q)
+        pos = 0
+        for n in cut:
+            jllm.call("jllm_hip_flash_attention_prefill_batched", out[pos:pos + n], q[pos:pos + n], k, v, H, KV, hd, hd,
+                      n, pos, 1.0 / np.sqrt(hd), int(int8), ks, vs, 0)
+            pos += n
+        assert pos == T
+        got = from_dev(out, np.uint16)
+        if want is None:
+            want = got
+        assert np.array_equal(got, want), cut
