@@ -1,8 +1,8 @@
 """Prefill attention kernel forms against float64: every (columns, waves) form of
 the launcher at its edges -- partial last blocks and key tiles, KV heads with 1 to
 16 query heads, every head size, INT8 and FP16 caches, windows, padded cache
-heads -- and V scales beyond the fp16-safe bound of the lazily moved softmax
-reference.  Bar: the output is fp16 (one rounding, 2^-11 of the value) of fp32
+heads -- V scales beyond the fp16-safe bound of the lazily moved softmax
+reference, and references that move in a state's later tiles.  Bar: the output is fp16 (one rounding, 2^-11 of the value) of fp32
 sums of ~22-bit probability products; 1e-3 of the largest output plus one fp16
 ulp of the value, the bar of the other attention tests."""
 import numpy as np
@@ -43,7 +43,7 @@ def _want(q, k, v, start, window, scale):
     (32, 8, 128, 0, False, 261, 800, 0, 1.0),       # the same form, fp16 cache
     (32, 8, 128, 0, True, 263, 900, 100, 1.0),      # window: short key ranges
     (32, 8, 128, 0, True, 261, 1200, 1100, 1.0),    # window: long key ranges
-    (32, 8, 128, 0, True, 40, 100, 0, 3e4),         # V scales beyond AP_VS_MAX (values near the fp16 limit)
+    (32, 8, 128, 0, True, 40, 100, 0, 3e4),         # V scales beyond AP_VS_MAX (values near the fp16 limit), one tile per state
     (8, 8, 64, 0, True, 70, 11, 0, 1.0),
     (12, 4, 96, 0, True, 50, 60, 0, 1.0),           # 3 heads per KV head: 30 of 32 columns live
     (12, 4, 96, 0, False, 50, 60, 20, 1.0),
@@ -148,3 +148,89 @@ def test_prefill_attention_bits_do_not_depend_on_the_cut(dev, H, KV, hd, int8, b
         if want is None:
             want = got
         assert np.array_equal(got, want), cut
+
+
+SLACK, STATES, TILE = 6.0, 8, 32      # AP_SLACK, AP_STATES and the keys of a tile
+
+
+def _replay(s2, vs, slack=SLACK):
+    """The lazily moved reference of one column over its base-2 scores: how often a
+    state's reference moved after its first tile, and the largest p * vs."""
+    moves, top = 0, 0.0
+    for u in range(STATES):
+        ref = None
+        for p0 in range(u * TILE, len(s2), STATES * TILE):
+            t = s2[p0:p0 + TILE]
+            if ref is None:
+                ref = t.max()
+            elif t.max() > ref + slack:
+                ref, moves = t.max(), moves + 1
+            top = max(top, float((np.exp2(t - ref) * vs[p0:p0 + TILE]).max()))
+    return moves, top
+
+
+# (N, start) on 32 / 8 heads: 8 waves, 4 waves (1024 keys), 64 columns
+FORMS = [(20, 1100), (300, 724), (300, 1100)]
+
+
+@pytest.mark.parametrize("N,start", FORMS)
+def test_prefill_attention_v_scales_under_a_lagging_reference(dev, N, start):
+    """V scales above AP_VS_MAX where a state's later tiles exceed its reference by
+    less than AP_SLACK: with the reference left behind, p * vs would pass the fp16
+    range (checked on the inputs), so these tiles have to take the exact maximum."""
+    print_case("attn_prefill_vs_lag", N, start)
+    H, KV, hd = 32, 8, 128
+    g = synth.rng(N + start)
+    ctx, scale = start + N, 1.0 / np.sqrt(hd)
+    q = (0.5 * (1.0 + 0.05 * g.standard_normal((N, H, hd)))).astype(np.float16)
+    k = (64 + g.integers(-8, 9, size=(ctx, KV, hd))).astype(np.int8)
+    # base-2 scores by the tile's place in its state: 0, then 5.5 (behind by less
+    # than the slack), 5, 11 (moves), 5, ...
+    target = np.array([0.02, 5.5, 5.0, 11.0, 5.0, 11.2])[np.arange(ctx) // (TILE * STATES)]
+    ks = np.repeat((target * np.log(2.0) / (0.5 * 64 * hd * scale)).astype(np.float32)[:, None], KV, 1)
+    v = g.integers(-12, 13, size=(ctx, KV, hd), dtype=np.int8)
+    vs = (2000.0 + 2000.0 * g.random((ctx, KV))).astype(np.float32)           # |v * vs| <= 48000
+    kf = k * ks[..., None].astype(np.float64)
+    s2 = kf[:, 0] @ q[-1, 0].astype(np.float64) * scale / np.log(2.0)
+    assert _replay(s2, vs[:, 0])[1] > 65504.0 and _replay(s2, vs[:, 0], 0.0)[1] < 65504.0
+    out = torch.empty(N * H * hd, dtype=torch.int16, device=dev)
+    jllm.call("jllm_hip_flash_attention_prefill_batched", out, to_dev(q.view(np.uint16)), to_dev(k), to_dev(v), H, KV, hd,
+              hd, N, start, scale, 1, to_dev(ks), to_dev(vs), 0)
+    got = f16_to_f64(from_dev(out, np.uint16)).reshape(N, H, hd)
+    want = _want(q.astype(np.float64), kf, v * vs[..., None].astype(np.float64), start, 0, scale)
+    err = np.abs(got - want)
+    assert np.all(err <= 1e-3 * np.abs(want).max() + np.abs(want) * 2 ** -10), float(err.max())
+
+
+@pytest.mark.parametrize("N,start", FORMS)
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+def test_prefill_attention_moved_reference(dev, hd, int8, N, start):
+    """Several tiles per state, whose maxima grow by more than 2^AP_SLACK from one to
+    the next (checked on the inputs) and fall again: the accumulators are rescaled
+    in mid-run and the K / V buffers reused, at every head size and cache type."""
+    print_case("attn_prefill_moved", hd, int8, N, start)
+    H, KV = 32, 8
+    g = synth.rng(hd + N + start)
+    ctx, scale = start + N, 1.0 / np.sqrt(hd)
+    q = g.standard_normal((N, H, hd)).astype(np.float16)
+    grow = np.array([1.0, 5.0, 2.0, 9.0, 3.0, 16.0])[np.arange(ctx) // (TILE * STATES)][:, None, None]
+    kr, vr = g.standard_normal((ctx, KV, hd)) * grow, g.standard_normal((ctx, KV, hd))
+    if int8:
+        ks, vs = (np.abs(a).max(-1).astype(np.float32) / np.float32(127) for a in (kr, vr))
+        k, v = (np.rint(a / b[..., None]).astype(np.int8) for a, b in ((kr, ks), (vr, vs)))
+        kf, vf = k * ks[..., None].astype(np.float64), v * vs[..., None].astype(np.float64)
+        args = [to_dev(k), to_dev(v), to_dev(ks), to_dev(vs)]
+    else:
+        k, v = kr.astype(np.float16), vr.astype(np.float16)
+        kf, vf = k.astype(np.float64), v.astype(np.float64)
+        args = [to_dev(k.view(np.uint16)), to_dev(v.view(np.uint16)), None, None]
+    s2 = kf[:, 0] @ q[-1, 0].astype(np.float64) * scale / np.log(2.0)
+    assert _replay(s2, np.ones(ctx))[0] >= STATES
+    out = torch.empty(N * H * hd, dtype=torch.int16, device=dev)
+    jllm.call("jllm_hip_flash_attention_prefill_batched", out, to_dev(q.view(np.uint16)), args[0], args[1], H, KV, hd, hd,
+              N, start, scale, int(int8), args[2], args[3], 0)
+    got = f16_to_f64(from_dev(out, np.uint16)).reshape(N, H, hd)
+    want = _want(q.astype(np.float64), kf, vf, start, 0, scale)
+    err = np.abs(got - want)
+    assert np.all(err <= 1e-3 * np.abs(want).max() + np.abs(want) * 2 ** -10), float(err.max())
