@@ -178,8 +178,7 @@ int prefill_attention(uint16_t* out, const uint16_t* q, const void* k, const voi
     a.out = out; a.q = q; a.k = k; a.v = v; a.ks = k_scales; a.vs = v_scales;
     a.counters = nullptr; a.part = nullptr;
     a.n_heads = n_heads; a.n_kv = n_kv_heads; a.head_dim = head_dim; a.cache_head_dim = cache_head_dim;
-    a.seq = start_pos + 1; a.window = window; a.n_splits = 1; a.scale = scale; a.tokens = N;
-    a.tq = 1; a.wsplit = 1;
+    a.seq = start_pos + 1; a.window = window; a.scale = scale; a.tokens = N;
     const bool q8 = quant && quantized && head_dim % 32 == 0;
     if (q8) { a.qcodes = quant->codes; a.qscl = quant->scl; a.q_npad = quant->npad; a.q_i8 = quant->i8 ? 1 : 0; }
     const int st2 = launch_status(attn_prefill_launch(a, kv_int8 != 0, (hipStream_t)stream), "attention prefill");

@@ -55,7 +55,7 @@ constexpr int XS = QK_K + 8;          // fp16 per staged token row (16 B pad aga
 // only its result.
 // The unpack is done by every wave for 64 tokens only, so it bounds the loop
 // next to the loads: with this fma and the qh bits taken at bit 4 (one shift
-// less per word) 9728 x 2560 at 300 tokens went 45.2 -> 42.6 us against a
+// less per word) 9728 x 2560 at 300 tokens went 43.8 -> 41.5 us against a
 // packed subtract and multiply, same bits.
 __device__ __forceinline__ h8q codes_h8(uint32_t w0, uint32_t w1, _Float16 sc, _Float16 nb) {
     const uint32_t hi = 0x64646464u;
@@ -87,7 +87,7 @@ __device__ __forceinline__ void load_a(ARegs& a, const uint8_t* blk, int kg) {
 // j the fp16 values [8 q, 8 q + 8) (q = t & 3): a load instruction of four
 // lanes covers 64 contiguous bytes of a row (with 128 contiguous bytes per
 // thread every instruction touched 64 separate lines, each line in eight
-// instructions: 9728 x 2560 at 300 tokens 43.5 us against 38.3 us).  The sums
+// instructions: 9728 x 2560 at 300 tokens 41.5 us against 35.7 us).  The sums
 // X_j then come from four lanes of eight values each instead of one chain of
 // 32: fp32 as before, a shorter chain.
 struct XRegs { u32x4q v[8]; };

@@ -18,7 +18,7 @@ constexpr int MMQ_TILE_THREADS = 256;
 // element, each to a line of its own -- the address unit and the L2's request
 // rate were the bound of the kernels' end (us: Q4_K 9728 x 2560 at N = 1261
 // 111.5 -> 92.6, at N = 33 21.3 -> 17.0; Q6_K 2560 x 9728 at N = 512 74.2 ->
-// 61.1; Q5_K 9728 x 2560 at N = 300 50.2 -> 44.0; same bits).
+// 61.1; Q5_K 9728 x 2560 at N = 300 49.5 -> 43.8; same bits).
 template <bool F32>
 constexpr int mmq_tile_bytes(int tokens) { return tokens * 132 * (F32 ? 4 : 2); }
 
