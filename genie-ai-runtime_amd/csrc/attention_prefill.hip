@@ -13,16 +13,15 @@
 
 namespace jllm_hip {
 
-// One workgroup of W waves per (KV head, block of tq tokens).  Its columns
+// One workgroup of AP_WAVES waves per (KV head, block of tq tokens).  Its columns
 // are the (token, head) pairs of the block -- column c = token tok0 + c / G,
 // head kvh * G + c % G -- in NG groups of 32, and every wave holds all of
-// them.  The 32-key tiles are dealt to AP_STATES = 8 softmax states, tile t to
-// state t % 8, which are combined in LDS in a fixed order: 8 waves hold one
-// each; of 4 waves each forms two, one after the other (wave w state w, then
-// w + 4).  So every form of the launch gives the same bits, and with them a
-// token's result does not depend on how a prompt is cut into calls, as long as
-// its window does not bind (where it does, the tiles start at the window start
-// of the block's first token).
+// them; the waves deal the 32-key tiles among themselves, tile t to wave
+// t % AP_WAVES, and their softmax states are combined in LDS in wave order.  The
+// number of waves is the same in every form of the launch, so a token's result
+// does not depend on how a prompt is cut into calls, bit for bit, as long as its
+// window does not bind (where it does, the tiles start at the window start of the
+// block's first token).
 //
 // Everything a tile needs after its loads stays in a wave's registers.  Lane
 // (li = lane & 31, lg = lane >> 5), MFMA elements v = 0..15 <-> index
@@ -45,11 +44,9 @@ namespace jllm_hip {
 // exponentials 9), and a 32-key x 64-column tile takes ~430 of them against
 // 1664 clocks of MFMA; hence the one-operation conversions below, the scores
 // formed relative to the reference (one fma), and two column groups per K / V
-// conversion.  32 / 8 heads x 128, INT8 KV, 512 tokens: at start 0 17.1 -> 12.8
-// us, at start 7680 166 -> 113 us (584 TFLOP/s of q.k and p.v products) against
+// conversion.  32 / 8 heads x 128, INT8 KV, 512 tokens: at start 0 17.1 -> 14.1
+// us, at start 7680 167 -> 115 us (580 TFLOP/s of q.k and p.v products) against
 // the form it replaces (P' through LDS, lane-per-row loads, exact maxima).
-// The second state of a wave costs the 4-wave form 0.9-1.1 us a call (11.7 us at
-// start 0 with one state per wave, whose bits followed the form).
 //
 // A column's softmax reference is not its running maximum but a value at most
 // AP_SLACK (in base 2) below it, so that the accumulators are rescaled only
@@ -59,7 +56,7 @@ namespace jllm_hip {
 // the fp16 range times 1/127) take the exact maximum.
 constexpr float AP_SLACK = 6.0f, AP_VS_MAX = 1000.0f;
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr int AP_STATES = 8;
+constexpr int AP_WAVES = 8;
 
 typedef __attribute__((address_space(3))) void ap_lds_void;
 
@@ -128,9 +125,10 @@ __device__ __forceinline__ void ap_split(float q0, float q1, uint32_t& hi, uint3
     lo = h2_bits(__builtin_convertvector((f32x2a{l0, l1}), half2_t));
 }
 
-template <bool INT8, int HD, int NG, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool INT8, int HD, int NG>
+__global__ __launch_bounds__(64 * AP_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_prefill_kernel(AttnArgs a) {
+    constexpr int W = AP_WAVES;
     constexpr int EB = INT8 ? 1 : 2;
     constexpr int hd = HD, half = HD / 2;
     constexpr int NDT = HD / 32;                        // 32-wide d chunks
@@ -145,11 +143,9 @@ void attn_prefill_kernel(AttnArgs a) {
     constexpr int Q_B = 32 * NG * QLD * 2, LOOP_B = Q_B + W * (2 * TILE_B + 256);
     constexpr int COMB_B = W * 32 * OLD * 4;
     constexpr int AREA_B = LOOP_B > COMB_B ? LOOP_B : COMB_B;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[AREA_B + (AP_STATES * 2 + 1) * NG * 32 * 4];
-    float (*sML)[NG][2][32] = (float (*)[NG][2][32])(smem + AREA_B);    // [state]: m, l of the columns
-    float (*sDen)[32] = (float (*)[32])(smem + AREA_B + AP_STATES * 2 * NG * 32 * 4);
-    constexpr bool TWO = W < AP_STATES;                 // a wave forms two states
-    static_assert(W == AP_STATES || 2 * W == AP_STATES, "states per wave");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[AREA_B + (W * 2 + 1) * NG * 32 * 4];
+    float (*sML)[NG][2][32] = (float (*)[NG][2][32])(smem + AREA_B);    // [wave]: m, l of its columns
+    float (*sDen)[32] = (float (*)[32])(smem + AREA_B + W * 2 * NG * 32 * 4);
 
     const int t = (int)threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -221,7 +217,7 @@ void attn_prefill_kernel(AttnArgs a) {
         if (INT8) scn = sp[(int64_t)min(p0 + li, seq - 1) * sc_row];
     };
     const int first = lo_pos + wv * AT_KEYS;
-    constexpr int stride = AP_STATES * AT_KEYS;
+    constexpr int stride = W * AT_KEYS;
     if (first < seq) { load_rows(a.k, sK, first, l); load_sc(first); load_rows(a.v, sV, first, l); }
 
     // the columns' q rows, shared by the waves (zeros past the live columns)
@@ -247,27 +243,12 @@ void attn_prefill_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < NDT; i++) acc[g][i] = f32x16{};
     }
-    // TWO: the wave's first state, once its second one has begun (until then: no keys)
-    bool second = false;
-    float m1[NG], l1[NG];
-    f32x16 acc1[NG][TWO ? NDT : 1];
-#pragma unroll
-    for (int g = 0; g < NG; g++) {
-        m1[g] = -FLT_MAX;
-        l1[g] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < (TWO ? NDT : 1); i++) acc1[g][i] = f32x16{};
-    }
     __syncthreads();
 
     int lane = l;
 #pragma unroll 1
-    for (int p0 = first; p0 < seq;) {
-        // the wave's next tile (the first of its second state after the last of its first)
-        int next = p0 + stride;
-        const bool turn2 = TWO && !second && next >= seq;
-        if (turn2) next = first + W * AT_KEYS;
-        const int n = min(AT_KEYS, seq - p0), pn = min(next, seq - 1);
+    for (int p0 = first; p0 < seq; p0 += stride) {
+        const int n = min(AT_KEYS, seq - p0), pn = min(p0 + stride, seq - 1);
         // (opaque per tile: the addresses formed from these few lane constants
         // would otherwise be hoisted and spilled)
         asm volatile("" : "+v"(kx), "+v"(vx), "+v"(lane));
@@ -440,36 +421,16 @@ void attn_prefill_kernel(AttnArgs a) {
         }
         ap_wait_lds();                                   // the V rows have been read
         load_rows(a.v, sV, pn, lane);
-        p0 = next;
-        if (TWO && turn2 && next < seq) {
-            second = true;
-#pragma unroll
-            for (int g = 0; g < NG; g++) {
-                m1[g] = none[g] == 0.0f ? run_m[g] : -FLT_MAX;
-                l1[g] = run_l[g];
-                run_m[g] = 0.0f;
-                none[g] = -FLT_MAX;
-                run_l[g] = 0.0f;
-#pragma unroll
-                for (int i = 0; i < (TWO ? NDT : 1); i++) { acc1[g][i] = acc[g][i]; acc[g][i] = f32x16{}; }
-            }
-        }
     }
     ap_wait_vm<0>();                                     // the rows fetched past the last tile have landed
 
-    // 5. the states combined per column:
-    // out = sum_u acc_u 2^(m_u - M) / sum_u l_u 2^(m_u - M), M = max_u m_u; the
-    // numerator as the sum over w < 4 of the sums of states w and w + 4
+    // 5. the waves' states combined per column, waves in order:
+    // out = sum_w acc_w 2^(m_w - M) / sum_w l_w 2^(m_w - M), M = max_w m_w
     if (lg == 0) {
 #pragma unroll
         for (int g = 0; g < NG; g++) {
-            const int u = TWO && second ? wv + W : wv;
-            sML[u][g][0][li] = none[g] == 0.0f ? run_m[g] : -FLT_MAX;
-            sML[u][g][1][li] = run_l[g];
-            if (TWO) {
-                sML[wv + W - (u - wv)][g][0][li] = m1[g];
-                sML[wv + W - (u - wv)][g][1][li] = l1[g];
-            }
+            sML[wv][g][0][li] = none[g] == 0.0f ? run_m[g] : -FLT_MAX;
+            sML[wv][g][1][li] = run_l[g];
         }
     }
     __syncthreads();                                     // (every wave has read its last q rows, too)
@@ -480,29 +441,20 @@ void attn_prefill_kernel(AttnArgs a) {
     for (int g = 0; g < NG; g++) {
         float M = sML[0][g][0][li];
 #pragma unroll
-        for (int u = 1; u < AP_STATES; u++) M = fmaxf(M, sML[u][g][0][li]);
-        const float f = __builtin_amdgcn_exp2f((none[g] == 0.0f ? run_m[g] : -FLT_MAX) - M);
-        const float f1 = TWO ? __builtin_amdgcn_exp2f(m1[g] - M) : 0.0f;
+        for (int u = 1; u < W; u++) M = fmaxf(M, sML[u][g][0][li]);
+        const float f = __builtin_amdgcn_exp2f(sML[wv][g][0][li] - M);
         if (wv == 0 && lg == 0) {
             float den = 0.0f;
 #pragma unroll
-            for (int u = 0; u < AP_STATES; u++) den += sML[u][g][1][li] * __builtin_amdgcn_exp2f(sML[u][g][0][li] - M);
+            for (int u = 0; u < W; u++) den += sML[u][g][1][li] * __builtin_amdgcn_exp2f(sML[u][g][0][li] - M);
             sDen[g][li] = den;
         }
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
-            for (int m4 = 0; m4 < 4; m4++) {
-                // (products and sum rounded one by one, as where two waves hold the states)
-#pragma clang fp contract(off)
-                f32x4a o;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    o[i] = acc[g][dt][4 * m4 + i] * f;
-                    if (TWO) o[i] += acc1[g][TWO ? dt : 0][4 * m4 + i] * f1;
-                }
-                *(f32x4a*)&sO[(wv * 32 + li) * OLD + 32 * dt + 8 * m4 + 4 * lg] = o;
-            }
+            for (int m4 = 0; m4 < 4; m4++)
+                *(f32x4a*)&sO[(wv * 32 + li) * OLD + 32 * dt + 8 * m4 + 4 * lg] =
+                    f32x4a{acc[g][dt][4 * m4] * f, acc[g][dt][4 * m4 + 1] * f, acc[g][dt][4 * m4 + 2] * f, acc[g][dt][4 * m4 + 3] * f};
         __syncthreads();
         // each thread: 8 consecutive d of a column
         const int gc = min(32, GC - 32 * g);
@@ -510,12 +462,8 @@ void attn_prefill_kernel(AttnArgs a) {
             const int cl = e / nd8, d0 = (e - cl * nd8) * 8, c = 32 * g + cl;
             f32x4a n0 = f32x4a{0.0f, 0.0f, 0.0f, 0.0f}, n1 = n0;
 #pragma unroll
-            for (int u = 0; u < AP_STATES / 2; u++) {
-                f32x4a h0 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0], h1 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0 + 4];
-                if (!TWO) {
-                    h0 += *(const f32x4a*)&sO[((u + AP_STATES / 2) * 32 + cl) * OLD + d0];
-                    h1 += *(const f32x4a*)&sO[((u + AP_STATES / 2) * 32 + cl) * OLD + d0 + 4];
-                }
+            for (int u = 0; u < W; u++) {
+                const f32x4a h0 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0], h1 = *(const f32x4a*)&sO[(u * 32 + cl) * OLD + d0 + 4];
 #pragma unroll
                 for (int i = 0; i < 4; i++) { n0[i] += h0[i]; n1[i] += h1[i]; }
             }
@@ -551,36 +499,25 @@ void attn_prefill_kernel(AttnArgs a) {
     }
 }
 
-// Column groups and waves of a workgroup, by the grid and the keys a block
-// sees; the results do not depend on it (32 / 8 heads x 128, INT8 KV, us for 32
-// columns x 4 waves / 32 x 8 / 64 x 8; N tokens at start):
-//   a grid of 32-column blocks that leaves CUs idle: 8 waves share a block's
-//   keys, however few (N = 33 at 0: 6.8 / 6.3 / 9.5; 32 at 1000: 18.1 / 13.0 /
-//   19.9; 128 at 4000: 50.5 / 36.1 / 54.4);
-//   short key ranges: 4 waves, two workgroups on a CU (512 at 0: 12.8 / 14.9 /
-//   14.3; 512 at 256: 16.5 / 18.7 / 17.4; 512 at 512: 20.9 / 22.4 / 20.8);
-//   else 64 columns, half the K / V conversions and reads per column (512 at
-//   1024: 29.4 / 30.1 / 27.6; 512 at 7680: 139 / 140 / 114).
-// FP16 caches, head sizes 32 to 96, 1 to 16 heads on each of 1 to 32 KV heads and
-// windows (some 80 calls in all) take a form within 7 % of their best one, except 512
-// tokens at 2000 with a window of 512 (17.6 / 19.5 / 15.8).
-enum { AP_1x4, AP_1x8, AP_2x8 };
-static int attn_prefill_form(const AttnArgs& a) {
-    const int tq1 = ATTN_MAX_COLUMNS / (a.n_heads / a.n_kv);
-    if ((int64_t)a.n_kv * ((a.tokens + tq1 - 1) / tq1) <= 256) return AP_1x8;
-    int64_t keys = (int64_t)a.seq - 1 + a.tokens;
-    if (a.window > 0 && keys > (int64_t)a.window + tq1) keys = (int64_t)a.window + tq1;
-    return keys <= 1024 ? AP_1x4 : AP_2x8;
-}
-
+// Column groups of a workgroup, by the grid: one where 32-column blocks leave
+// CUs idle, else two, with half the K / V conversions and reads per column (32 /
+// 8 heads x 128, INT8 KV, us for 32 / 64 columns; N tokens at start: 33 at 0 6.2 /
+// 9.4; 32 at 1000 13.0 / 19.7; 256 at 512 11.6 / 16.6; 300 at 724 21.7 / 19.7; 512
+// at 0 14.8 / 14.1; 512 at 7680 142 / 115).  The same side is faster for FP16
+// caches, head sizes 32 to 96, 1 to 16 heads on each of 1 to 32 KV heads and
+// windows of 100 to 1500 keys (80 calls).
+// Four waves of 32 columns, two workgroups on a CU, were faster below ~500 keys
+// (512 at 0 11.6, at 256 15.5 against 17.2) and are not used: the bits would follow
+// the form, and with it the cut of a prompt.  Four waves that form the eight
+// states two each: 13.8 and 17.5.
 template <bool INT8, int HD>
 static void attn_prefill_go(AttnArgs& a, hipStream_t st) {
-    const int form = attn_prefill_form(a);
-    a.tq = (form == AP_2x8 ? 2 : 1) * ATTN_MAX_COLUMNS / (a.n_heads / a.n_kv);
+    const int tq1 = ATTN_MAX_COLUMNS / (a.n_heads / a.n_kv);
+    const bool one = (int64_t)a.n_kv * ((a.tokens + tq1 - 1) / tq1) <= 256;
+    a.tq = one ? tq1 : 2 * ATTN_MAX_COLUMNS / (a.n_heads / a.n_kv);
     const dim3 grid(a.n_kv, 1, (a.tokens + a.tq - 1) / a.tq);
-    if (form == AP_1x4)      hipLaunchKernelGGL((attn_prefill_kernel<INT8, HD, 1, 4>), grid, dim3(64 * 4), 0, st, a);
-    else if (form == AP_1x8) hipLaunchKernelGGL((attn_prefill_kernel<INT8, HD, 1, 8>), grid, dim3(64 * 8), 0, st, a);
-    else                     hipLaunchKernelGGL((attn_prefill_kernel<INT8, HD, 2, 8>), grid, dim3(64 * 8), 0, st, a);
+    if (one) hipLaunchKernelGGL((attn_prefill_kernel<INT8, HD, 1>), grid, dim3(64 * AP_WAVES), 0, st, a);
+    else     hipLaunchKernelGGL((attn_prefill_kernel<INT8, HD, 2>), grid, dim3(64 * AP_WAVES), 0, st, a);
 }
 
 hipError_t attn_prefill_launch(AttnArgs a, bool kv_int8, hipStream_t st) {

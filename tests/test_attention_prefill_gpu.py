@@ -1,4 +1,4 @@
-"""Prefill attention kernel forms against float64: every (columns, waves) form of
+"""Prefill attention kernel forms against float64: every form of
 the launcher at its edges -- partial last blocks and key tiles, KV heads with 1 to
 16 query heads, every head size, INT8 and FP16 caches, windows, padded cache
 heads -- V scales beyond the fp16-safe bound of the lazily moved softmax
@@ -36,14 +36,14 @@ def _want(q, k, v, start, window, scale):
 @pytest.mark.parametrize("H,KV,hd,pad,int8,N,start,window,vs_mul", [
     (32, 8, 128, 0, True, 1, 0, 0, 1.0),            # one key
     (32, 8, 128, 0, True, 7, 25, 0, 1.0),           # one partial block, keys end inside a tile
-    (32, 8, 128, 0, True, 256, 33, 0, 1.0),         # 256 blocks: 8 waves
-    (32, 8, 128, 0, True, 257, 0, 0, 1.0),          # 257 blocks: 4 waves
-    (32, 8, 128, 0, True, 300, 724, 0, 1.0),        # 1024 keys: 4 waves
-    (32, 8, 128, 0, True, 300, 725, 0, 1.0),        # 1025 keys: 64 columns
+    (32, 8, 128, 0, True, 256, 33, 0, 1.0),         # 256 blocks: 32 columns
+    (32, 8, 128, 0, True, 257, 0, 0, 1.0),          # 257 blocks: 64 columns
+    (32, 8, 128, 0, True, 300, 724, 0, 1.0),        # 64 columns, 1024 keys
+    (32, 8, 128, 0, True, 300, 725, 0, 1.0),        # a partial last tile
     (32, 8, 128, 0, False, 261, 800, 0, 1.0),       # the same form, fp16 cache
     (32, 8, 128, 0, True, 263, 900, 100, 1.0),      # window: short key ranges
     (32, 8, 128, 0, True, 261, 1200, 1100, 1.0),    # window: long key ranges
-    (32, 8, 128, 0, True, 40, 100, 0, 3e4),         # V scales beyond AP_VS_MAX (values near the fp16 limit), one tile per state
+    (32, 8, 128, 0, True, 40, 100, 0, 3e4),         # V scales beyond AP_VS_MAX (values near the fp16 limit), one tile per wave
     (8, 8, 64, 0, True, 70, 11, 0, 1.0),
     (12, 4, 96, 0, True, 50, 60, 0, 1.0),           # 3 heads per KV head: 30 of 32 columns live
     (12, 4, 96, 0, False, 50, 60, 20, 1.0),
@@ -80,7 +80,7 @@ def test_prefill_attention_forms(dev, H, KV, hd, pad, int8, N, start, window, vs
 
 
 @pytest.mark.parametrize("hd", [32, 64, 96, 128])
-@pytest.mark.parametrize("N,start", [(20, 700), (300, 200), (300, 900)])    # 8 waves, 4 waves, 64 columns
+@pytest.mark.parametrize("N,start", [(20, 700), (300, 200), (300, 900)])    # 32 columns, 64 columns
 @pytest.mark.parametrize("with_ks,with_vs", [(False, False), (True, False), (False, True)])
 def test_prefill_attention_without_scales(dev, hd, N, start, with_ks, with_vs):
     """INT8 caches whose k_scales and / or v_scales are NULL (= 1.0), several key
@@ -150,7 +150,7 @@ def test_prefill_attention_bits_do_not_depend_on_the_cut(dev, H, KV, hd, int8, b
         assert np.array_equal(got, want), cut
 
 
-SLACK, STATES, TILE = 6.0, 8, 32      # AP_SLACK, AP_STATES and the keys of a tile
+SLACK, STATES, TILE = 6.0, 8, 32      # AP_SLACK, AP_WAVES (a state each) and the keys of a tile
 
 
 def _replay(s2, vs, slack=SLACK):
@@ -169,7 +169,7 @@ def _replay(s2, vs, slack=SLACK):
     return moves, top
 
 
-# (N, start) on 32 / 8 heads: 8 waves, 4 waves (1024 keys), 64 columns
+# (N, start) on 32 / 8 heads: 32 columns, 64 columns
 FORMS = [(20, 1100), (300, 724), (300, 1100)]
 
 
