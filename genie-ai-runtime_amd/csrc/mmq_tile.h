@@ -38,27 +38,34 @@ __device__ __forceinline__ void mmq_put_tile(uint8_t* T, int tl, int r0, const m
 }
 
 // the tile's rows row0 .. row0 + 127 (< M) of tokens col0 .. (< N) to y [N][M]
-// (fp32: to the partials of this range of K, blockIdx.y); 256 threads
+// (fp32: to the partials of this range of K, blockIdx.y); 256 threads.  Where a
+// 16-byte piece would not be aligned (M or y), consecutive lanes store
+// consecutive elements.
 template <bool F32>
 __device__ __forceinline__ void mmq_store_tile(void* y, const uint8_t* T, int row0, int col0, int tokens, int M, int N) {
     constexpr int PR = F32 ? 4 : 8, NPR = 128 / PR;    // rows of a 16-byte piece, pieces per token
     const int64_t base = F32 ? (int64_t)blockIdx.y * N * M : 0;
-    const bool vec = M % PR == 0 && ((uintptr_t)y & 15u) == 0;
-    for (int e = threadIdx.x; e < tokens * NPR; e += MMQ_TILE_THREADS) {
-        const int tl = e / NPR, r = row0 + (e % NPR) * PR, tok = col0 + tl;
-        if (tok >= N || r >= M) continue;
-        const int64_t at = base + (int64_t)tok * M + r;
-        if (F32) {
-            const mt_f32x4 v = *(const mt_f32x4*)((const float*)T + tl * 132 + (r - row0));
-            if (vec) *(mt_f32x4*)((float*)y + at) = v;
-            else for (int i = 0; i < PR && r + i < M; i++) ((float*)y)[at + i] = v[i];
-        } else {
-            const uint16_t* t = (const uint16_t*)T + tl * 132 + (r - row0);
-            const mt_u32x2 a = *(const mt_u32x2*)t, b = *(const mt_u32x2*)(t + 4);
-            const mt_u32x4 v = mt_u32x4{a.x, a.y, b.x, b.y};
-            if (vec) *(mt_u32x4*)((uint16_t*)y + at) = v;
-            else for (int i = 0; i < PR && r + i < M; i++) ((uint16_t*)y)[at + i] = (uint16_t)(v[i >> 1] >> (16 * (i & 1)));
+    if (M % PR == 0 && ((uintptr_t)y & 15u) == 0) {
+        for (int e = threadIdx.x; e < tokens * NPR; e += MMQ_TILE_THREADS) {
+            const int tl = e / NPR, r = row0 + (e % NPR) * PR, tok = col0 + tl;
+            if (tok >= N || r >= M) continue;
+            const int64_t at = base + (int64_t)tok * M + r;
+            if (F32) {
+                *(mt_f32x4*)((float*)y + at) = *(const mt_f32x4*)((const float*)T + tl * 132 + (r - row0));
+            } else {
+                const uint16_t* t = (const uint16_t*)T + tl * 132 + (r - row0);
+                const mt_u32x2 a = *(const mt_u32x2*)t, b = *(const mt_u32x2*)(t + 4);
+                *(mt_u32x4*)((uint16_t*)y + at) = mt_u32x4{a.x, a.y, b.x, b.y};
+            }
         }
+        return;
+    }
+    const int r = threadIdx.x & 127;
+    if (row0 + r >= M) return;
+    for (int tl = threadIdx.x >> 7; tl < min(tokens, N - col0); tl += MMQ_TILE_THREADS / 128) {
+        const int64_t at = base + (int64_t)(col0 + tl) * M + row0 + r;
+        if (F32) ((float*)y)[at] = ((const float*)T)[tl * 132 + r];
+        else     ((uint16_t*)y)[at] = ((const uint16_t*)T)[tl * 132 + r];
     }
 }
 
