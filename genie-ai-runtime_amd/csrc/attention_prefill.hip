@@ -21,7 +21,9 @@ namespace jllm_hip {
 // number of waves is the same in every form of the launch, so a token's result
 // does not depend on how a prompt is cut into calls, bit for bit, as long as its
 // window does not bind (where it does, the tiles start at the window start of the
-// block's first token).
+// block's first token).  A value of V or a V scale that is not finite is the
+// exception: masked keys enter the products with probability 0, so it reaches
+// every token of its block, the earlier ones too.
 //
 // Everything a tile needs after its loads stays in a wave's registers.  Lane
 // (li = lane & 31, lg = lane >> 5), MFMA elements v = 0..15 <-> index
@@ -40,9 +42,9 @@ namespace jllm_hip {
 // The K rows of the wave's next tile are fetched as soon as Q.K^T has read the
 // current ones, the V rows after P.V: one LDS buffer each.
 // What bounds it: VALU issue.  With MFMAs in flight a SIMD issues one VALU
-// operation per ~5 clocks whatever its number of waves (conversions 6,
-// exponentials 9), and a 32-key x 64-column tile takes ~430 of them against
-// 1664 clocks of MFMA; hence the one-operation conversions below, the scores
+// operation per 5.3 clocks whatever its number of waves (exponentials 9.3:
+// microbench/issue_rates.hip), and a 32-key x 64-column tile takes ~440 of them in
+// the loop, ~2500 clocks against 1664 of MFMA; hence the one-operation conversions below, the scores
 // formed relative to the reference (one fma), and two column groups per K / V
 // conversion.  32 / 8 heads x 128, INT8 KV, 512 tokens: at start 0 17.1 -> 14.1
 // us, at start 7680 167 -> 115 us (580 TFLOP/s of q.k and p.v products) against
